@@ -37,6 +37,7 @@ SOURCES = [
     "qconv_dot4.hip",
     "gemm_i32.hip",
     "conv_f32.hip",
+    "conv_f32_split.hip",
     "grad_noalloc.hip",
     "qconv_qi32.hip",
     "qconv_qi32_band.hip",

@@ -19,6 +19,8 @@
 //   - Two chunks are in flight per thread.  Every pass of the loop issues the same loads:
 //     taps outside the image, values past kdim and rows past M or Kg read a valid address
 //     and are zeroed (or never stored), so the compiler's load counters stay exact.
+//   It serves what the split-bf16 kernel (conv_f32_split.hip) leaves to it: one-tap layers of a
+//   short reduction, few output channels at a stride, dilation below 1, the dx of a blocked filter.
 //   The sum order differs from the reference's sequential fp32 loop; results agree within
 //   the reference's own check (verify_tensors with abs 1e-4 / rel 1e-3, main.cpp:306-316).
 //
@@ -1424,6 +1426,8 @@ bool f32_igemm_eligible(const Geom& g, const BlockGeom& bg, const void* x, const
 
 hipError_t launch_f32_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                             int bias_mode, float* y, hipStream_t stream) {
+  hipError_t e;
+  if (launch_f32_split(g, bg, x, w, bias, bias_mode, y, false, stream, &e)) return e;
   return f32_igemm_launch(g, bg, fprop_regions(bg), x, w, bias, bias_mode, y, false, stream);
 }
 
@@ -1455,6 +1459,8 @@ bool f32_bprop_igemm_eligible(const Geom& g, const BlockGeom& bg, const void* dy
 hipError_t launch_f32_bprop_igemm(const Geom& g, const BlockGeom& bg, const float* dy, const float* w, float* dx,
                                   hipStream_t stream) {
   const Geom b = f32_bprop_as_fprop(g);
+  hipError_t e;
+  if (bg.By * bg.Bx == 1 && launch_f32_split(b, dense_blocks(b), dy, w, nullptr, 0, dx, true, stream, &e)) return e;
   return f32_igemm_launch(b, bg, bprop_regions(b, bg), dy, w, nullptr, 0, dx, true, stream);
 }
 

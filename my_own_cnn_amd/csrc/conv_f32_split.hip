@@ -1,0 +1,686 @@
+// fp32 NHWC convolution on the bf16 matrix cores, without losing fp32 accuracy: the forward pass
+// and, read with the flipped, channel-transposed filter, the dx of a stride-1 convolution.
+//
+// Arithmetic.  Each operand is split into three bf16 numbers, x = x0 + x1 + x2 (round to nearest
+// even at each step: 8 + 8 + 8 significant bits hold all 24 of an fp32 value of magnitude 2^-110
+// and more).  A product is the six terms x2 w0, x0 w2, x1 w1, x0 w1, x1 w0, x0 w0; the dropped
+// ones are below 2^-26 of it.  The terms of 32 reduction values sum from zero in that order, and
+// the sum is added to the fp32 accumulator.  Error against 64 bits, K = 576 / 4608 normal
+// inputs: 0.9e-7 / 2.3e-7 relative, where a chain of v_mfma_f32_16x16x4f32 gives 4.4e-7 / 1.2e-6
+// (one rounding of the running sum per 32 products, not per 4).  Six
+// v_mfma_f32_16x16x32_bf16 issue in 0.38 of the time of the eight v_mfma_f32_16x16x4f32 they
+// replace; a loop of them alone sustains 1680 TFLOP/s on this card, 280 of them the convolution's.
+// Inputs the split does not carry are found at run time and their whole tile is computed again
+// with v_mfma_f32_16x16x4f32: a nonzero value below 2^-110 (checked as the values are staged), and
+// anything that makes a stored result infinite or NaN (an infinite or NaN input, or a value that
+// rounds up to a bf16 infinity).
+//
+// Work.  A workgroup computes a tile of ti images x th x tw output positions (at most
+// 16 NSEG WM) and 32 WN channels of one group; wave (wm, wn) computes 16 NSEG of the positions
+// x 32 channels.  The reduction runs over chunks of `co` octets (8 channels) and, within a
+// chunk, over the R S co (tap, octet) pairs, 4 to a K-block (one pair per lane group):
+//   - A: the tile's input halo of the chunk is read once from memory, split once, and kept in LDS
+//     as [octet][halo position][3 pieces] of 16 bytes; every tap reads it at its own offset.  The
+//     implicit GEMM gathers (and would split) each value once per tap.
+//   - B: the filter values of SO octets a stage, [octet][channel][3 pieces], double-buffered.
+// The next stage's filter values and the next chunk's halo are in flight in registers while a
+// stage's MFMAs run.
+//
+// Measured (us; before: the fp32 implicit GEMM of conv_f32.hip): 32 x 56 x 56, 64 -> 64 3x3 54-58
+// (110), its dx 58 (122); 32 x 28 x 28, 128 -> 256 97 (207), dx 97 (226), 2 x 4 filter blocks 93
+// (199); 16 x 64 x 64 dilated 32 (57); four groups of 32 64 (111); one 56 x 56 image 14.6 (30.6).
+// Bound by the matrix instructions and the power they draw: with everything but the MFMAs and
+// their LDS reads taken out the 28 x 28 dx still took 67 us; the filter's split and stores cost 8,
+// its loads 8 and the halo 4.  The 56 x 56 layer loses a further 9 us per workgroup at its start
+// and end (halo load and split, stores), which a second workgroup per CU hides only in part.
+
+#include "qconv_device.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace miq {
+namespace {
+
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+constexpr int kSplitUnits = 4;             // halo (position, octet) pairs per thread
+constexpr int kSplitLds = 160 * 1024;      // bytes per CU
+constexpr int kSplitMaxOct = 1024;         // (tap, octet) pairs of a chunk
+constexpr unsigned kSmall2 = (17u << 24) - 1u;  // 2 * bits(2^-110) - 1
+
+struct SplitArgs {
+  const float* x;
+  const float* w;
+  const float* bias;
+  float* y;
+  Geom g;
+  int kdim;        // R * S * Cg
+  int tn;          // channel tiles per group
+  int tiles;       // pixel tiles * tn per region
+  int nty, ntx;    // tile rows and columns per region
+  int ti, th, tw;  // images, rows and columns of a tile
+  int hh, hw;      // halo rows and columns per image
+  int twp;         // tile columns a row of positions takes (tw, or tw rounded up to 16)
+  int hp;          // halo positions, ti * hh * hw
+  int hps;         // slots per octet plane (a multiple of 16, >= hp)
+  int co;          // octets per chunk
+  int ash;         // extra slots before every second octet plane
+  int lgh;         // log2(co / 2) for 2, 4 or 8 octets, else -1
+  int nchunk;
+  int noct;        // R * S * co
+  int nst;         // stages per chunk
+  int ow_taps, ow_cg;  // transposed filter: R * S and channels per group of the original
+  int rx, nreg, rh, rw;  // output regions (the filter blocks) of rh x rw positions, rx per row
+  int By, Bx, bias_mode;
+  FastDivM fd_tn, fd_tiles, fd_reg, fd_rx, fd_ntx, fd_nty, fd_co, fd_s, fd_hw, fd_hhw, fd_twp, fd_thw;
+};
+
+struct Split8 {
+  v4u p[3];
+};
+
+// Eight fp32 values as three bf16 each; `mn` collects the smallest 2 * bits - 1 (zero wraps to the
+// largest unsigned value).
+__device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, unsigned& mn) {
+  Split8 out;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const v2f v = j < 2 ? v2f{lo[2 * j], lo[2 * j + 1]} : v2f{hi[2 * j - 4], hi[2 * j - 3]};
+    const unsigned u0 = (__builtin_bit_cast(unsigned, static_cast<float>(v[0])) << 1) - 1u;
+    const unsigned u1 = (__builtin_bit_cast(unsigned, static_cast<float>(v[1])) << 1) - 1u;
+    mn = min(mn, min(u0, u1));
+    const v2b h = __builtin_convertvector(v, v2b);
+    const v2f r1 = v2f{v[0] - static_cast<float>(h[0]), v[1] - static_cast<float>(h[1])};
+    const v2b m = __builtin_convertvector(r1, v2b);
+    const v2f r2 = v2f{r1[0] - static_cast<float>(m[0]), r1[1] - static_cast<float>(m[1])};
+    const v2b l = __builtin_convertvector(r2, v2b);
+    out.p[0][j] = __builtin_bit_cast(unsigned, h);
+    out.p[1][j] = __builtin_bit_cast(unsigned, m);
+    out.p[2][j] = __builtin_bit_cast(unsigned, l);
+  }
+  return out;
+}
+
+// 16 and 4 bytes at byte offset voff + soff of a buffer; zero where voff is past its 2^31 - 1 bytes
+__device__ __forceinline__ v4f buffer_load16(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
+  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+__device__ __forceinline__ float buffer_load4(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
+}
+
+__device__ __forceinline__ int f32s_slot(int row, int g) { return 4 * row + (g ^ (((row >> 3) & 1) << 1)); }
+
+template <bool TRANS, int NSEG, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a) {
+  constexpr int NT = 64 * WM * WN;
+  constexpr int BM = 16 * NSEG * WM;
+  constexpr int BN = 32 * WN;
+  constexpr int SO = 2 * WM < 4 ? 4 : 2 * WM;  // filter octets per stage
+  constexpr int BU = SO * BN / NT;             // filter (channel, octet) pairs per thread
+  constexpr int BSH = 16 / SO;                 // extra slots before every second filter octet
+  constexpr int BSZ = 3 * (SO * BN + BSH * SO / 2);  // 16-byte slots of a filter buffer
+  static_assert(BU >= 1 && BU * NT == SO * BN && (SO == 4 || SO == 8), "whole filter stages");
+  extern __shared__ v4u lds[];
+  const Geom& g = a.g;
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wn = wave % WN;
+  const int wm = wave / WN;
+
+  v4u* const sA = lds;                                  // 3 * co * hps slots
+  v4u* const sB = lds + 3 * (a.co * a.hps + 8);         // two filter buffers
+  int* const tab = reinterpret_cast<int*>(sB + 2 * BSZ);  // nst * SO entries, then the flag
+
+  const int lin = xcd_tile(blockIdx.x, gridDim.x);
+  const int gr = fdiv(lin, a.fd_tiles);  // group * regions + region
+  const int rem = lin - gr * a.tiles;
+  const int grp = fdiv(gr, a.fd_reg);
+  const int reg = gr - grp * a.nreg;
+  const int rgy = fdiv(reg, a.fd_rx);
+  const int rgx = reg - rgy * a.rx;
+  const int tmi = fdiv(rem, a.fd_tn);
+  const int n0 = (rem - tmi * a.tn) * BN;  // first channel of the group
+  const int tq = fdiv(tmi, a.fd_ntx);
+  const int tx0 = (tmi - tq * a.ntx) * a.tw;
+  const int tim = fdiv(tq, a.fd_nty);
+  const int ty0 = (tq - tim * a.nty) * a.th;
+  const int img0 = tim * a.ti;
+  const int row0 = rgy * a.rh, col0 = rgx * a.rw;
+  const int h0 = (row0 + ty0) * g.sh - g.ph;  // input position of the halo's origin
+  const int w0 = (col0 + tx0) * g.sw - g.pw;
+
+  // a tile position m: image, row and column in the tile, and whether it is an output
+  auto decode = [&](int m, int& im, int& lr, int& lc) -> bool {
+    im = fdiv(m, a.fd_thw);
+    const int p = m - im * (a.th * a.twp);
+    lr = fdiv(p, a.fd_twp);
+    lc = p - lr * a.twp;
+    return im < a.ti && img0 + im < g.N && lc < a.tw && ty0 + lr < a.rh && tx0 + lc < a.rw;
+  };
+
+  // LDS slot (in units of 48 bytes) of octet oc's plane.  ds_read_b128 serves lane quads of both
+  // 16-lane groups of a half-wave in one cycle, so the planes of an even and the next odd octet
+  // lie a multiple of 16 apart; ds_write_b128 serves 8 consecutive lanes, which stage octets of
+  // one parity: those planes are `ash` further on each.
+  auto plane = [&](int oc) { return oc * a.hps + (oc >> 1) * a.ash; };
+  // halo units of this thread: byte offset from the tile's first image (kNone: reads zero), LDS
+  // slot and octet
+  constexpr unsigned kNone = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t rx =
+      make_rsrc(a.x + static_cast<size_t>(img0) * g.H * g.W * g.C + static_cast<size_t>(grp) * g.Cg, 0x7fffffff);
+  unsigned aoff[kSplitUnits];
+  unsigned aput[kSplitUnits];  // slot | octet << 20
+#pragma unroll
+  for (int j = 0; j < kSplitUnits; ++j) {
+    const int u = t + NT * j;
+    int px, oc;
+    if (a.lgh >= 0) {
+      const int l = u & 15, h = 1 << a.lgh;
+      oc = ((l & (h - 1)) << 1) | (l >> 3);
+      px = ((u >> 4) << (3 - a.lgh)) + ((l & 7) >> a.lgh);
+    } else {
+      px = fdiv(u, a.fd_co);
+      oc = u - px * a.co;
+    }
+    const int im = fdiv(px, a.fd_hhw);
+    const int p = px - im * (a.hh * a.hw);
+    const int hr = fdiv(p, a.fd_hw);
+    const int hi = h0 + hr;
+    const int wi = w0 + p - hr * a.hw;
+    const bool in = px < a.hp;
+    const bool ok = in && img0 + im < g.N && hi >= 0 && hi < g.H && wi >= 0 && wi < g.W;
+    aoff[j] = ok ? 4u * (static_cast<unsigned>((im * g.H + hi) * g.W + wi) * g.C + 8 * oc) : kNone;
+    aput[j] = in ? static_cast<unsigned>(3 * (plane(oc) + px)) | static_cast<unsigned>(oc) << 20 : ~0u;
+  }
+  // filter units: octet boct[j] of a stage, LDS slot, byte offset of the channel's row (TRANS: of
+  // the channel)
+  int boct[BU], bslot[BU];
+  unsigned boff[BU];
+  const int nblk = a.By * a.Bx;
+  const int ko_stride = a.ow_taps * a.ow_cg;
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(
+      TRANS ? a.w + static_cast<size_t>(grp) * g.Cg * ko_stride
+            : a.w + (static_cast<size_t>(grp) * g.Kg * nblk + reg) * a.kdim, 0x7fffffff);
+#pragma unroll
+  for (int j = 0; j < BU; ++j) {
+    const int u = t + NT * j;
+    constexpr int H = SO / 2;
+    const int r = TRANS ? u % BN : (u >> 4) * (8 / H) + ((u & 7) / H);
+    boct[j] = TRANS ? u / BN : (((u & (H - 1)) << 1) | ((u >> 3) & 1));
+    bslot[j] = 3 * (boct[j] * BN + (boct[j] >> 1) * BSH + r);
+    const int kr = min(n0 + r, g.Kg - 1);
+    boff[j] = 4u * (TRANS ? static_cast<unsigned>(kr) : static_cast<unsigned>(kr * nblk) * a.kdim);
+  }
+  // LDS offset of each (tap, octet) pair's halo values, relative to a position's slot
+  for (int o = t; o < a.nst * SO; o += NT) {
+    const int tap = fdiv(o, a.fd_co);
+    const int r = fdiv(tap, a.fd_s);
+    const int off = plane(o - tap * a.co) + r * g.dh * a.hw + (tap - r * g.S) * g.dw;
+    tab[o] = o < a.noct ? 48 * off : 0;
+  }
+  int* const flag = tab + a.nst * SO;
+  if (t == 0) *flag = 0;
+
+  // the tile's segments of 16 positions, spread evenly over the WM rows of waves: this wave's
+  // first, how many are its own, and whether that is NSEG (else it computes NSEG - 1 and keeps its own)
+  const int segs = (a.ti * a.th * a.twp + 15) >> 4;
+  const int each = segs / WM, extra = segs - each * WM;
+  const int seg0 = wm * each + min(wm, extra);
+  const int own = each + (wm < extra ? 1 : 0);
+  const bool whole = own >= NSEG;
+  const int m0 = 16 * seg0 + (lane & 15);
+  int pbase[NSEG];  // byte offset of this lane's positions
+#pragma unroll
+  for (int i = 0; i < NSEG; ++i) {
+    int im, lr, lc;
+    const bool ok = decode(m0 + 16 * i, im, lr, lc);
+    pbase[i] = ok ? 48 * ((im * a.hh + lr * g.sh) * a.hw + lc * g.sw) : 0;
+  }
+
+  v4f va[kSplitUnits][2];
+  v4f vb[BU][2];
+  unsigned mn = 0xffffffffu;
+  const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
+  auto load_a = [&](int c) {
+    const int c0 = 8 * a.co * c;
+#pragma unroll
+    for (int j = 0; j < kSplitUnits; ++j) {
+      const int left = g.Cg - c0 - 8 * static_cast<int>(aput[j] >> 20);
+      va[j][0] = buffer_load16(rx, left >= 4 ? aoff[j] : kNone, 4 * c0);
+      va[j][1] = buffer_load16(rx, left >= 8 ? aoff[j] + 16u : kNone, 4 * c0);
+    }
+  };
+  auto store_a = [&]() {
+#pragma unroll
+    for (int j = 0; j < kSplitUnits; ++j) {
+      if (aput[j] != ~0u) {
+        const Split8 s = split8(va[j][0], va[j][1], mn);
+        v4u* const d = sA + (aput[j] & 0xfffffu);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) d[p] = s.p[p];
+      }
+    }
+  };
+  auto load_b = [&](int c, int s) {
+    const int c0 = 8 * a.co * c;
+#pragma unroll
+    for (int j = 0; j < BU; ++j) {
+      const int o = SO * s + boct[j];
+      const int tap = fdiv(o, a.fd_co);
+      const int ch = c0 + 8 * (o - tap * a.co);
+      const int left = o < a.noct ? g.Cg - ch : 0;
+      if constexpr (TRANS) {
+        const unsigned off = boff[j] + 4u * (ch * ko_stride + (a.ow_taps - 1 - tap) * a.ow_cg);
+        const unsigned o0 = left >= 4 ? off : kNone, o1 = left >= 8 ? off : kNone;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vb[j][0][e] = buffer_load4(rw, o0, 4 * e * ko_stride);
+          vb[j][1][e] = buffer_load4(rw, o1, 4 * (e + 4) * ko_stride);
+        }
+      } else {
+        const unsigned off = boff[j] + 4u * (tap * g.Cg + ch);
+        vb[j][0] = buffer_load16(rw, left >= 4 ? off : kNone, 0);
+        vb[j][1] = buffer_load16(rw, left >= 8 ? off + 16u : kNone, 0);
+      }
+    }
+  };
+  auto store_b = [&](int buf) {  // the values of the last load_b
+#pragma unroll
+    for (int j = 0; j < BU; ++j) {
+      const Split8 sp = split8(vb[j][0], vb[j][1], mn);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) sB[buf * BSZ + bslot[j] + p] = sp.p[p];
+    }
+  };
+
+  v4f acc[2][NSEG];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < NSEG; ++i) acc[j][i] = zero;
+
+  const char* const bA = reinterpret_cast<const char*>(sA);
+  const char* const bB = reinterpret_cast<const char*>(sB) + 48 * (32 * wn + (lane & 15) + BN * q + BSH * (q >> 1));
+  // Stages in order over the chunks, for a wave of NS segments: the filter values of stage i + 1
+  // are split and stored, and those of stage i + 2 fetched, inside stage i.  A K-block runs in
+  // steps of up to two segments; a step's fragments are read while the step before it computes.
+  // The six products of a step sum from zero, smallest first, and are added to the accumulators.
+  int lc = 0, ls = 0;  // stage of the next load_b
+  auto fetch = [&]() {
+    load_b(lc, ls);
+    if (++ls == a.nst) {
+      ls = 0;
+      lc = min(lc + 1, a.nchunk - 1);  // past the end: loaded, never used
+    }
+  };
+  auto run = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    constexpr int HALVES = (NS + 1) / 2;       // steps per K-block
+    constexpr int STEPS = SO / 4 * HALVES;     // steps per stage
+    int buf = 0;
+    for (int c = 0; c < a.nchunk; ++c) {
+      const bool more = c + 1 < a.nchunk;
+      for (int s = 0; s < a.nst; ++s) {
+        int ao[SO / 4];
+#pragma unroll
+        for (int kb = 0; kb < SO / 4; ++kb) ao[kb] = tab[SO * s + 4 * kb + q];
+        const char* const bs = bB + 16 * buf * BSZ;
+        v8b fa[2][2][3], fb[2][2][3];
+        auto read = [&](int st) {
+          const int kb = st / HALVES, i0 = 2 * (st % HALVES);
+          if (i0 == 0) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int p = 0; p < 3; ++p)
+                fb[kb & 1][j][p] = *reinterpret_cast<const v8b*>(bs + 16 * p + 48 * (4 * kb * BN + 2 * kb * BSH + 16 * j));
+          }
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            if (i0 + i < NS) {
+#pragma unroll
+              for (int p = 0; p < 3; ++p)
+                fa[st & 1][i][p] = *reinterpret_cast<const v8b*>(bA + pbase[i0 + i] + ao[kb] + 16 * p);
+            }
+        };
+        auto step = [&](auto stc) {
+          constexpr int st = decltype(stc)::value;
+          constexpr int kb = st / HALVES, i0 = 2 * (st % HALVES);
+          if constexpr (st + 1 < STEPS) read(st + 1);
+          __builtin_amdgcn_sched_barrier(0x276);  // the reads above, the MFMAs below; the rest may move
+          v4f z[2][2];
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            constexpr int kw[6] = {2, 0, 1, 1, 0, 0}, kx[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              if (i0 + i < NS) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                  z[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kb & 1][j][kw[k]], fa[st & 1][i][kx[k]],
+                                                                    k == 0 ? zero : z[j][i], 0, 0, 0);
+              }
+          }
+          if constexpr (st == 0) {
+            store_b(buf ^ 1);
+            fetch();
+            if (s == 0) load_a(more ? c + 1 : c);
+          }
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            if (i0 + i < NS) {
+#pragma unroll
+              for (int j = 0; j < 2; ++j) acc[j][i0 + i] += z[j][i];
+            }
+        };
+        read(0);
+        step(std::integral_constant<int, 0>{});
+        if constexpr (HALVES > 1) step(std::integral_constant<int, 1>{});
+        if constexpr (SO > 4) {
+          if (SO * s + 4 < a.noct) {  // uniform: a second K-block
+            step(std::integral_constant<int, HALVES>{});
+            if constexpr (HALVES > 1) step(std::integral_constant<int, HALVES + 1>{});
+          }
+        }
+        __syncthreads();
+        buf ^= 1;
+      }
+      if (more) {
+        store_a();
+        __syncthreads();
+      }
+    }
+  };
+  fetch();
+  load_a(0);
+  store_b(0);
+  fetch();
+  store_a();
+  __syncthreads();
+  // both arms run the same barriers
+  if (whole) run(std::integral_constant<int, NSEG>{});
+  else run(std::integral_constant<int, NSEG - 1>{});
+
+  bool bad = mn < kSmall2;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < NSEG; ++i) {
+      int im, lr, lc;
+      const bool ok = i < own && decode(m0 + 16 * i, im, lr, lc);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        bad |= ok && !(__builtin_fabsf(acc[j][i][e]) <= 3.4028234663852886e38f);
+      }
+    }
+  if (bad) *flag = 1;
+  __syncthreads();
+  if (*flag != 0) {
+    // the tile again with fp32 MFMAs: per tap, 16 channels a step, gathered into LDS
+    constexpr int UR = BM * 4 / NT;
+    v4f* const fA = reinterpret_cast<v4f*>(lds);
+    v4f* const fB = fA + BM * 4;
+    int uh[UR], uw[UR];
+    const float* ux[UR];
+#pragma unroll
+    for (int k = 0; k < UR; ++k) {
+      int im, lr, lc;
+      const bool ok = decode((t + NT * k) >> 2, im, lr, lc);
+      uh[k] = ok ? h0 + lr * g.sh : INT32_MIN / 2;
+      uw[k] = w0 + lc * g.sw;
+      ux[k] = a.x + static_cast<size_t>(ok ? img0 + im : 0) * g.H * g.W * g.C + static_cast<size_t>(grp) * g.Cg;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < NSEG; ++i) acc[j][i] = zero;
+    for (int tap = 0; tap < g.R * g.S; ++tap) {
+      const int r = fdiv(tap, a.fd_s);
+      const int s = tap - r * g.S;
+      for (int c0 = 0; c0 < g.Cg; c0 += 16) {
+        __syncthreads();  // the previous step's reads (and the flag's)
+        const int ch = c0 + 4 * (t & 3);
+#pragma unroll
+        for (int k = 0; k < UR; ++k) {
+          const int hi = uh[k] + r * g.dh, wi = uw[k] + s * g.dw;
+          const bool ok = ch < g.Cg && hi >= 0 && hi < g.H && wi >= 0 && wi < g.W;
+          const v4f v = *reinterpret_cast<const v4f*>(ok ? ux[k] + (static_cast<size_t>(hi) * g.W + wi) * g.C + ch : a.x);
+          fA[f32s_slot((t + NT * k) >> 2, t & 3)] = ok ? v : zero;
+        }
+        for (int u = t; u < BN * 4; u += NT) {
+          const int kr = min(n0 + (u >> 2), g.Kg - 1);
+          const int cb = c0 + 4 * (u & 3);
+          v4f v = zero;
+          if (cb < g.Cg) {
+            if constexpr (TRANS) {
+              const float* p = a.w + (static_cast<size_t>(grp) * g.Cg + cb) * ko_stride +
+                               static_cast<size_t>(a.ow_taps - 1 - tap) * a.ow_cg + kr;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] = p[e * ko_stride];
+            } else {
+              v = *reinterpret_cast<const v4f*>(a.w + (static_cast<size_t>(grp * g.Kg + kr) * nblk + reg) * a.kdim +
+                                                static_cast<size_t>(tap) * g.Cg + cb);
+            }
+          }
+          fB[f32s_slot(u >> 2, u & 3)] = v;
+        }
+        __syncthreads();
+        v4f fb[2], fa[NSEG];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[j] = fB[f32s_slot(32 * wn + 16 * j + (lane & 15), q)];
+#pragma unroll
+        for (int i = 0; i < NSEG; ++i) fa[i] = fA[f32s_slot(min(m0 + 16 * i, BM - 1), q)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < NSEG; ++i)
+              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][k], fa[i][k], acc[j][i], 0, 0, 0);
+      }
+    }
+  }
+
+  // lane (c = lane % 16, q): position c of each segment, channels 4 q .. 4 q + 3 of each 16
+  const bool vec = (g.K & 3) == 0 && (g.Kg & 3) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15u) == 0;
+  const int bias_y = a.bias_mode == 0 ? rgy : 0;
+  const int bias_x = a.bias_mode == 0 ? rgx : 0;
+#pragma unroll
+  for (int i = 0; i < NSEG; ++i) {
+    int im, lr, lc;
+    if (i >= own || !decode(m0 + 16 * i, im, lr, lc)) continue;
+    const size_t pix = (static_cast<size_t>(img0 + im) * g.Ho + row0 + ty0 + lr) * g.Wo + col0 + tx0 + lc;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int ch = n0 + 32 * wn + 16 * j + 4 * q;
+      float* yp = a.y + pix * g.K + static_cast<size_t>(grp) * g.Kg + ch;
+      v4f r = acc[j][i];
+      if (!TRANS && a.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = grp * g.Kg + min(ch + e, g.Kg - 1);
+          r[e] = __fadd_rn(r[e], a.bias[(static_cast<size_t>(k) * a.By + bias_y) * a.Bx + bias_x]);
+        }
+      }
+      if (vec && ch + 3 < g.Kg) {
+        *reinterpret_cast<v4f*>(yp) = r;
+        store_gap(r);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (ch + e < g.Kg) yp[e] = r[e];
+      }
+    }
+  }
+}
+
+// Tile of one launch variant, and its estimated time.
+struct SplitPlan {
+  int variant;  // index into kVariants, -1: none fits
+  int ti, th, tw, twp, hh, hw, hp, hps, co, ash, nchunk, noct, nst;
+  int nty, ntx, nti, tn;
+  size_t lds;
+  long long blocks;
+  double cost;
+};
+
+struct SplitVariant {
+  int nseg, wm, wn;
+};
+constexpr SplitVariant kVariants[] = {{4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {4, 4, 1}};
+
+// Estimated cycles of a launch: rounds of workgroups over the 256 CUs x (K-blocks at the MFMA rate
+// of a wave's tile, the staged values, a fixed start and end).
+void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int th, int tw, int twp,
+              SplitPlan* best) {
+  const SplitVariant& V = kVariants[v];
+  const int nt = 64 * V.wm * V.wn, bn = 32 * V.wn, so = std::max(4, 2 * V.wm);
+  SplitPlan p{};
+  p.variant = v;
+  p.ti = ti; p.th = th; p.tw = tw; p.twp = twp;
+  p.hh = (th - 1) * g.sh + (g.R - 1) * g.dh + 1;
+  p.hw = (tw - 1) * g.sw + (g.S - 1) * g.dw + 1;
+  const long long hp = static_cast<long long>(ti) * p.hh * p.hw;
+  if (hp > kSplitUnits * nt || static_cast<double>(ti) * g.H * g.W * g.C * 4 >= 2147483647.0) return;
+  p.hp = static_cast<int>(hp);
+  p.nty = (rh + th - 1) / th;
+  p.ntx = (rw + tw - 1) / tw;
+  p.nti = (g.N + ti - 1) / ti;
+  p.tn = (g.Kg + bn - 1) / bn;
+  p.blocks = nreg * g.G * p.nty * p.ntx * static_cast<long long>(p.nti) * p.tn;
+  const int oct = (g.Cg + 7) / 8;
+  int tried = 0;
+  for (const int want : {8, 6, 4, 3, 2, 1}) {  // octets of a chunk, evened out over the chunks
+    if (want > oct && want != 8 && tried != 0) continue;
+    const int chunks = (oct + want - 1) / want;
+    const int co = (oct + chunks - 1) / chunks;
+    if (co == tried) continue;
+    tried = co;
+    if (co == 1 && oct > 1) continue;  // a K-block of four taps: its fragment reads conflict in the banks
+    const long long noct = static_cast<long long>(g.R) * g.S * co;
+    if (hp * co > kSplitUnits * nt || noct > kSplitMaxOct) continue;
+    p.co = co;
+    p.nchunk = (oct + co - 1) / co;
+    p.noct = static_cast<int>(noct);
+    p.nst = (p.noct + so - 1) / so;
+    p.hps = (p.hp + 15) & ~15;
+    p.ash = co >= 6 ? 2 : (co >= 4 ? 4 : 0);
+    const int bsz = 3 * (so * bn + (16 / so) * so / 2);
+    p.lds = static_cast<size_t>(3 * (co * p.hps + 8) + 2 * bsz) * 16 + static_cast<size_t>(p.nst * so + 1) * 4;
+    if (p.lds > kSplitLds) continue;
+    const int per_cu = std::max(1, std::min<int>({static_cast<int>(kSplitLds / p.lds), 8 / (V.wm * V.wn), 4}));
+    const double kb = static_cast<double>(p.nchunk) * ((p.noct + 3) / 4);
+    const double mfma = kb * V.nseg * 12 * 16.0 * V.wm * V.wn / 4;  // SIMD cycles of a workgroup
+    const double stage = p.nchunk * (static_cast<double>(p.hp) * co + static_cast<double>(p.nst) * so * bn) * 60.0 / 64;
+    const double wg = mfma * 1.25 + stage * 0.7 + 2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
+    const double rounds = std::ceil(static_cast<double>(p.blocks) / (256.0 * per_cu)) * per_cu;
+    p.cost = std::min(rounds, static_cast<double>(p.blocks) / 256.0 + 0.5 * per_cu) * wg;
+    if (p.blocks < 256) p.cost = wg;
+    if (best->variant < 0 || p.cost < best->cost) *best = p;
+  }
+}
+
+// The tile of a launch, or variant -1 where the fp32 implicit GEMM is the faster kernel (measured
+// on a 32 x 56 x 56 layer unless a size is given): with one tap nothing is read twice from the
+// halo and a short reduction leaves the split unpaid (1x1 128 -> 256: 100 against 89 us; 512 -> 128
+// at 14 x 14: 24.5 against 28; transposed 256 -> 64: 43 against 59), and at most 32 output channels
+// at a stride give too few MFMAs per halo value (112 x 112, 32 -> 32: 39 against 35 us, 32 -> 64:
+// 24 against 31).
+SplitPlan make_plan(const Geom& g, int rh, int rw, long long nreg, bool transposed) {
+  SplitPlan best{};
+  best.variant = -1;
+  if (g.dh <= 0 || g.dw <= 0 || g.sh <= 0 || g.sw <= 0) return best;
+  if (g.R * g.S == 1 && g.Cg < (transposed ? 128 : 256)) return best;
+  if (g.Kg <= 32 && (g.sh > 1 || g.sw > 1)) return best;
+  // 32-bit byte offsets: into a group's filter (every block of it) and into an image
+  if (static_cast<double>(std::max(g.Kg, g.Cg)) * nreg * g.R * g.S * std::max(g.Kg, g.Cg) * 4 >= 2147483647.0 ||
+      static_cast<double>(g.H) * g.W * g.C * 4 >= 2147483647.0) {
+    return best;
+  }
+  for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
+    if (kVariants[v].wn == 1 && g.Kg > 32) continue;
+    if (kVariants[v].wn == 2 && g.Kg <= 32) continue;
+    const int bm = 16 * kVariants[v].nseg * kVariants[v].wm;
+    int last = 0;
+    for (int j = 1; j <= 12; ++j) {
+      const int tw = (rw + j - 1) / j;
+      if (tw > bm || tw == last) continue;
+      last = tw;
+      int th = std::min(rh, bm / tw);
+      th = (rh + (rh + th - 1) / th - 1) / ((rh + th - 1) / th);  // even rows of tiles
+      const int ti = th == rh && tw == rw ? std::max(1, std::min(g.N, bm / (th * tw))) : 1;
+      const int tw16 = (tw + 15) & ~15;  // rows of whole segments: no segment wraps into the next row
+      if (tw16 != tw && ti * th * tw16 <= bm) consider(g, rh, rw, nreg, v, ti, th, tw, tw16, &best);
+      else consider(g, rh, rw, nreg, v, ti, th, tw, tw, &best);
+      if (tw <= 8) break;
+    }
+  }
+  return best;
+}
+
+template <bool TRANS, int NSEG, int WM, int WN>
+hipError_t launch_variant(const SplitArgs& a, const SplitPlan& p, hipStream_t stream) {
+  if (p.lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&f32_split_kernel<TRANS, NSEG, WM, WN>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kSplitLds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((f32_split_kernel<TRANS, NSEG, WM, WN>), dim3(static_cast<unsigned>(p.blocks)),
+                     dim3(64 * WM * WN), p.lds, stream, a);
+  return hipGetLastError();
+}
+
+template <bool TRANS>
+hipError_t launch_split(const SplitArgs& a, const SplitPlan& p, hipStream_t stream) {
+  switch (p.variant) {
+    case 0: return launch_variant<TRANS, 4, 4, 2>(a, p, stream);
+    case 1: return launch_variant<TRANS, 4, 2, 2>(a, p, stream);
+    case 2: return launch_variant<TRANS, 2, 2, 2>(a, p, stream);
+    default: return launch_variant<TRANS, 4, 4, 1>(a, p, stream);
+  }
+}
+
+}  // namespace
+
+bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
+                      int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err) {
+  const int nreg = bg.By * bg.Bx;
+  const SplitPlan p = make_plan(g, bg.bho, bg.bwo, nreg, transposed);
+  if (p.variant < 0 || p.blocks <= 0 || p.blocks > (1LL << 22)) return false;
+  SplitArgs a;
+  a.x = x; a.w = w; a.bias = bias; a.y = y; a.g = g;
+  a.kdim = g.R * g.S * g.Cg;
+  a.tn = p.tn;
+  a.tiles = static_cast<int>(static_cast<long long>(p.nty) * p.ntx * p.nti * p.tn);
+  a.nty = p.nty; a.ntx = p.ntx;
+  a.ti = p.ti; a.th = p.th; a.tw = p.tw; a.hh = p.hh; a.hw = p.hw; a.hp = p.hp; a.hps = p.hps;
+  a.twp = p.twp; a.ash = p.ash; a.lgh = p.co == 2 ? 0 : (p.co == 4 ? 1 : (p.co == 8 ? 2 : -1));
+  a.co = p.co; a.nchunk = p.nchunk; a.noct = p.noct; a.nst = p.nst;
+  a.ow_taps = g.R * g.S;
+  a.ow_cg = g.Kg;
+  a.rx = bg.Bx; a.nreg = nreg; a.rh = bg.bho; a.rw = bg.bwo;
+  a.By = bg.By; a.Bx = bg.Bx; a.bias_mode = bias_mode;
+  a.fd_tn = fastdiv_m(a.tn);
+  a.fd_tiles = fastdiv_m(a.tiles);
+  a.fd_reg = fastdiv_m(nreg);
+  a.fd_rx = fastdiv_m(a.rx);
+  a.fd_ntx = fastdiv_m(a.ntx);
+  a.fd_nty = fastdiv_m(a.nty);
+  a.fd_co = fastdiv_m(a.co);
+  a.fd_s = fastdiv_m(g.S);
+  a.fd_hw = fastdiv_m(a.hw);
+  a.fd_hhw = fastdiv_m(a.hh * a.hw);
+  a.fd_twp = fastdiv_m(a.twp);
+  a.fd_thw = fastdiv_m(a.th * a.twp);
+  *err = transposed ? launch_split<true>(a, p, stream) : launch_split<false>(a, p, stream);
+  return true;
+}
+
+}  // namespace miq

@@ -198,6 +198,11 @@ inline BlockGeom dense_blocks(const Geom& g) { return BlockGeom{1, 1, g.Ho, g.Wo
 bool f32_igemm_eligible(const Geom& g, const BlockGeom& bg, const void* x, const void* w, std::string* why);
 hipError_t launch_f32_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                             int bias_mode, float* y, hipStream_t stream);
+// The same forward pass on the bf16 matrix cores, each operand split into three bf16 numbers
+// (fp32 accuracy); `transposed`: the dx of a stride-1 convolution with a plain filter, g and bg
+// those of f32_bprop_as_fprop.  False when no tile of the shape fits (nothing is launched).
+bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
+                      int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err);
 hipError_t launch_f32_direct(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                              int bias_mode, float* y, hipStream_t stream);
 // fp32 depthwise (C/groups == K/groups == 1, C % 4 == 0, R*S*C <= 8192, 16-byte aligned x and y),

@@ -1,0 +1,119 @@
+"""The fp32 convolution on split bf16 operands: sizes at the edges of its tiles, channel octets,
+stages and chunks, and the inputs that it hands back to the fp32 instructions.
+
+Bound against 64 bits: a K-block of 32 reduction values is summed with a few fp32 roundings of
+its own and added with one more, and the dropped products are below 2^-26 of each term, so every
+output is within (K / 32 + 16) 2^-23 of the sum of |x w| (a factor two in hand)."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+import my_own_cnn_amd as M
+
+pytestmark = pytest.mark.gpu
+
+# (n, h, w, c, k, r, s, (ph, pw, sh, sw, dh, dw, groups))
+CASES = [
+    (1, 5, 4, 4, 33, 3, 3, (1, 1, 1, 1, 1, 1, 1)),       # one half octet, a channel past the tile
+    (2, 17, 19, 12, 40, 3, 3, (1, 1, 1, 1, 1, 1, 1)),    # octet tail
+    (3, 33, 29, 20, 48, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (5, 7, 7, 72, 65, 3, 3, (1, 1, 1, 1, 1, 1, 1)),      # several images per tile, an uneven chunk
+    (37, 3, 3, 64, 36, 3, 3, (1, 1, 1, 1, 1, 1, 1)),     # images past the last tile
+    (2, 30, 57, 64, 64, 3, 3, (0, 2, 1, 1, 1, 1, 1)),
+    (1, 23, 21, 96, 66, 5, 3, (2, 1, 1, 1, 2, 3, 1)),    # dilation, K not a multiple of 4
+    (2, 25, 31, 32, 96, 3, 3, (1, 1, 2, 2, 1, 1, 1)),    # stride
+    (1, 40, 18, 24, 64, 7, 7, (3, 3, 2, 1, 1, 1, 1)),
+    (2, 14, 15, 80, 64, 3, 3, (1, 1, 1, 1, 1, 1, 4)),    # groups
+    (1, 1, 3, 256, 300, 1, 1, (0, 0, 1, 1, 1, 1, 1)),    # one tap
+    (1, 9, 130, 264, 32, 1, 1, (0, 0, 1, 1, 1, 1, 1)),
+    (1, 6, 6, 16, 32, 3, 3, (3, 3, 1, 1, 1, 1, 1)),      # padding past the filter's reach
+]
+
+
+def conv64(x, w, conv):
+    ph, pw, sh, sw, dh, dw, g = conv
+    y = F.conv2d(x.double().permute(0, 3, 1, 2), w.double().permute(0, 3, 1, 2), padding=(ph, pw), stride=(sh, sw),
+                 dilation=(dh, dw), groups=g)
+    return y.permute(0, 2, 3, 1)
+
+
+def data(case, seed):
+    n, h, w, c, k, r, s, conv = case
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn((n, h, w, c), generator=gen), torch.randn((k, r, s, c // conv[6]), generator=gen))
+
+
+def check(got, want, mag, kdim):
+    err = (got.double() - want).abs()
+    assert bool((err <= (kdim / 32 + 16) * 2.0 ** -23 * mag + 1e-300).all()), float((err / mag.clamp(min=1e-300)).max())
+
+
+@pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
+def test_forward_and_dx(device, case):
+    n, h, w, c, k, r, s, conv = case
+    x, wt = data(case, 7 + CASES.index(case))
+    y = M.conv2d_nhwc_f32(x.to(device), wt.to(device), padding=conv[:2], stride=conv[2:4], dilation=conv[4:6], groups=conv[6])
+    check(y.cpu(), conv64(x, wt, conv), conv64(x.abs(), wt.abs(), conv), wt[0].numel())
+    if conv[2] != 1 or conv[3] != 1 or (k // conv[6]) % 4:
+        return
+    xg = x.double().requires_grad_()
+    dy = torch.randn(y.shape, generator=torch.Generator().manual_seed(1))
+    want, = torch.autograd.grad(conv64(xg, wt, conv), xg, dy.double())
+    mag, = torch.autograd.grad(conv64(xg, wt.abs(), conv), xg, dy.double().abs())
+    dx = torch.full(x.shape, 7.0, device=device)
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, n, h, w, c, r, s, k, conv)
+    check(dx.cpu(), want, mag, r * s * k // conv[6])
+
+
+@pytest.mark.parametrize("grid", [(2, 3), (4, 2)])
+def test_blocked_forward(device, grid):
+    n, h, w, c, k = 3, 16, 18, 40, 70
+    by, bx = grid
+    gen = torch.Generator().manual_seed(3)
+    x, wt = torch.randn((n, h, w, c), generator=gen), torch.randn((k, by, bx, 3, 3, c), generator=gen)
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    y = torch.empty((n, h, w, k), device=device)
+    M.launch_block_fprop_nhwc(x.to(device), wt.to(device), y, n, h, w, c, 3, 3, k,
+                              M.BlockConv2DParams(M.Conv2DParams(*conv), by, bx))
+    for i in range(by):
+        for j in range(bx):
+            rows, cols = slice(i * h // by, (i + 1) * h // by), slice(j * w // bx, (j + 1) * w // bx)
+            f = wt[:, i, j].contiguous()
+            check(y[:, rows, cols].cpu(), conv64(x, f, conv)[:, rows, cols], conv64(x.abs(), f.abs(), conv)[:, rows, cols], 9 * c)
+
+
+def test_infinite_and_nan_inputs(device):
+    x, wt = data((2, 20, 20, 32, 40, 3, 3, (1, 1, 1, 1, 1, 1, 1)), 5)
+    x[0, 3, 4, 5], x[0, 10, 12, 7], x[1, 19, 19, 31], x[1, 0, 0, 0] = float("inf"), float("nan"), float("-inf"), 3.4e38
+    y = M.conv2d_nhwc_f32(x.to(device), wt.to(device), padding=1).cpu()
+    # image by tap: a tap outside the image multiplies by nothing
+    want = conv64(torch.nan_to_num(x, nan=0.0, posinf=0.0, neginf=0.0), wt, (1, 1, 1, 1, 1, 1, 1))
+    for im, r, c, ch, v in ((0, 3, 4, 5, float("inf")), (0, 10, 12, 7, float("nan")), (1, 19, 19, 31, float("-inf"))):
+        for i in range(3):
+            for j in range(3):
+                hh, ww = r - i + 1, c - j + 1
+                if 0 <= hh < 20 and 0 <= ww < 20:
+                    want[im, hh, ww] += v * wt[:, i, j, ch].double()
+    over = want.abs() > 3.4028235677973366e38
+    want = torch.where(over & want.isfinite(), torch.sign(want) * float("inf"), want)
+    assert torch.equal(y.isnan(), want.isnan())
+    fin = want.isfinite()
+    assert torch.equal(y[~fin & ~want.isnan()].double(), want[~fin & ~want.isnan()])
+    assert bool(((y[fin].double() - want[fin]).abs() <= 1e-4 + 1e-5 * want[fin].abs()).all())
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -112, 2.0 ** -126, 2.0 ** -140])
+def test_small_inputs(device, scale):
+    case = (1, 12, 12, 32, 36, 3, 3, (1, 1, 1, 1, 1, 1, 1))
+    x, wt = data(case, 6)
+    x, wt = x * scale, wt * 2.0 ** 30
+    y = M.conv2d_nhwc_f32(x.to(device), wt.to(device), padding=1).cpu()
+    check(y, conv64(x, wt, case[7]), conv64(x.abs(), wt.abs(), case[7]), 9 * 32)
+    dx = torch.empty_like(x, device=device)
+    dy = torch.randn((1, 12, 12, 36), generator=torch.Generator().manual_seed(2)) * scale
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, 1, 12, 12, 32, 3, 3, 36, case[7])
+    xg = x.double().requires_grad_()
+    want, = torch.autograd.grad(conv64(xg, wt, case[7]), xg, dy.double())
+    mag, = torch.autograd.grad(conv64(xg, wt.abs(), case[7]), xg, dy.double().abs())
+    check(dx.cpu(), want, mag, 9 * 36)

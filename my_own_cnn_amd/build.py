@@ -38,6 +38,7 @@ SOURCES = [
     "gemm_i32.hip",
     "conv_f32.hip",
     "conv_f32_split.hip",
+    "conv_f32_split_grad.hip",
     "grad_noalloc.hip",
     "qconv_qi32.hip",
     "qconv_qi32_band.hip",

@@ -854,7 +854,9 @@ __global__ void __launch_bounds__(kDirectThreads) f32_grad_direct_kernel(const f
   dw[e] = acc;
 }
 
-// dw on the matrix cores: dw[g Kg + k][j] = sum over pixels p of dy[p][g Kg + k] * col[p][j],
+// dw on the fp32 matrix cores, for what the split-bf16 kernel (conv_f32_split_grad.hip) leaves to
+// it (channel counts that are not multiples of 4, unaligned tensors, the float-atomic form, a few
+// shapes it is slower on): dw[g Kg + k][j] = sum over pixels p of dy[p][g Kg + k] * col[p][j],
 // j = (r, s, ci) the filter column, col the implicit im2col of x.  A workgroup of 8 waves
 // computes 128 columns x 64 channels over its share of the pixels (chunks of 16), with the
 // fprop kernel's staging, fragment layout and pipeline; the pixel range is split over
@@ -1224,10 +1226,23 @@ void launch_sum_parts(const float* part, float* dw, long long count, long long n
 
 }  // namespace
 
+namespace {
+
+// Partial tiles the workspace holds: the implicit GEMM's splits, or, where those are more than half
+// the CUs, up to one per CU for the split-bf16 kernel while 32 MiB hold them (the caller's scratch
+// array of miq_grad_nhwc_f32_noalloc).
+long long grad_max_splits(const Geom& g, const BlockGeom& bg) {
+  const long long splits = grad_split(g, bg, true).splits;
+  const long long slice = static_cast<long long>(g.K) * bg.By * bg.Bx * g.R * g.S * g.Cg * 4;
+  return splits > 128 ? std::max(splits, std::min(256LL, (32LL << 20) / std::max(slice, 1LL))) : splits;
+}
+
+}  // namespace
+
 size_t f32_grad_igemm_workspace(const Geom& g, const BlockGeom& bg) {
-  const GradSplit sp = grad_split(g, bg, true);
-  if (sp.splits <= 1) return 0;
-  return static_cast<size_t>(sp.splits) * g.K * bg.By * bg.Bx * g.R * g.S * g.Cg * sizeof(float);
+  const long long splits = grad_max_splits(g, bg);
+  if (splits <= 1) return 0;
+  return static_cast<size_t>(splits) * g.K * bg.By * bg.Bx * g.R * g.S * g.Cg * sizeof(float);
 }
 
 hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw,
@@ -1241,6 +1256,15 @@ hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float
   a.tiles = ((a.kdim + kF32BM - 1) / kF32BM) * a.tn;
   a.gt = a.tiles * g.G * bg.By * bg.Bx;
   const GradSplit sp = grad_split(g, bg, ordered);
+  if (ordered) {
+    long long splits = 0;
+    hipError_t e;
+    if (launch_f32_split_grad(g, bg, x, dy, dw, ws, grad_max_splits(g, bg), stream, &splits, &e)) {
+      if (e == hipSuccess && splits > 1)
+        launch_sum_parts(ws, dw, static_cast<long long>(g.K) * bg.By * bg.Bx * a.kdim, splits, stream);
+      return e != hipSuccess ? e : hipGetLastError();
+    }
+  }
   a.cps = sp.cps;
   a.fd_tn = fastdiv_m(a.tn);
   a.fd_tiles = fastdiv_m(a.tiles);

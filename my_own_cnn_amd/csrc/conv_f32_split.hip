@@ -34,7 +34,7 @@
 // its loads 8 and the halo 4.  The 56 x 56 layer loses a further 9 us per workgroup at its start
 // and end (halo load and split, stores), which a second workgroup per CU hides only in part.
 
-#include "qconv_device.h"
+#include "f32_split.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -42,15 +42,8 @@
 namespace miq {
 namespace {
 
-typedef __bf16 v8b __attribute__((ext_vector_type(8)));
-typedef __bf16 v2b __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-
 constexpr int kSplitUnits = 4;             // halo (position, octet) pairs per thread
-constexpr int kSplitLds = 160 * 1024;      // bytes per CU
 constexpr int kSplitMaxOct = 1024;         // (tap, octet) pairs of a chunk
-constexpr unsigned kSmall2 = (17u << 24) - 1u;  // 2 * bits(2^-110) - 1
 
 struct SplitArgs {
   const float* x;
@@ -78,40 +71,6 @@ struct SplitArgs {
   int By, Bx, bias_mode;
   FastDivM fd_tn, fd_tiles, fd_reg, fd_rx, fd_ntx, fd_nty, fd_co, fd_s, fd_hw, fd_hhw, fd_twp, fd_thw;
 };
-
-struct Split8 {
-  v4u p[3];
-};
-
-// Eight fp32 values as three bf16 each; `mn` collects the smallest 2 * bits - 1 (zero wraps to the
-// largest unsigned value).
-__device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, unsigned& mn) {
-  Split8 out;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const v2f v = j < 2 ? v2f{lo[2 * j], lo[2 * j + 1]} : v2f{hi[2 * j - 4], hi[2 * j - 3]};
-    const unsigned u0 = (__builtin_bit_cast(unsigned, static_cast<float>(v[0])) << 1) - 1u;
-    const unsigned u1 = (__builtin_bit_cast(unsigned, static_cast<float>(v[1])) << 1) - 1u;
-    mn = min(mn, min(u0, u1));
-    const v2b h = __builtin_convertvector(v, v2b);
-    const v2f r1 = v2f{v[0] - static_cast<float>(h[0]), v[1] - static_cast<float>(h[1])};
-    const v2b m = __builtin_convertvector(r1, v2b);
-    const v2f r2 = v2f{r1[0] - static_cast<float>(m[0]), r1[1] - static_cast<float>(m[1])};
-    const v2b l = __builtin_convertvector(r2, v2b);
-    out.p[0][j] = __builtin_bit_cast(unsigned, h);
-    out.p[1][j] = __builtin_bit_cast(unsigned, m);
-    out.p[2][j] = __builtin_bit_cast(unsigned, l);
-  }
-  return out;
-}
-
-// 16 and 4 bytes at byte offset voff + soff of a buffer; zero where voff is past its 2^31 - 1 bytes
-__device__ __forceinline__ v4f buffer_load16(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
-  return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
-__device__ __forceinline__ float buffer_load4(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
 
 __device__ __forceinline__ int f32s_slot(int row, int g) { return 4 * row + (g ^ (((row >> 3) & 1) << 1)); }
 
@@ -172,7 +131,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   auto plane = [&](int oc) { return oc * a.hps + (oc >> 1) * a.ash; };
   // halo units of this thread: byte offset from the tile's first image (kNone: reads zero), LDS
   // slot and octet
-  constexpr unsigned kNone = 0x80000000u;
   const __amdgpu_buffer_rsrc_t rx =
       make_rsrc(a.x + static_cast<size_t>(img0) * g.H * g.W * g.C + static_cast<size_t>(grp) * g.Cg, 0x7fffffff);
   unsigned aoff[kSplitUnits];

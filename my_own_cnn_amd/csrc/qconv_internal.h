@@ -229,6 +229,11 @@ bool f32_grad_igemm_eligible(const Geom& g, const BlockGeom& bg, std::string* wh
 size_t f32_grad_igemm_workspace(const Geom& g, const BlockGeom& bg);
 hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw,
                                  float* ws, bool ordered, hipStream_t stream);
+// The same dw on the bf16 matrix cores (each operand split into three bf16 numbers), with at most
+// max_splits partial tiles in `ws`, which the caller sums in order; one split writes dw.  False
+// when the shape does not fit (nothing is launched).
+bool launch_f32_split_grad(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw, float* ws,
+                           long long max_splits, hipStream_t stream, long long* splits, hipError_t* err);
 // Bias gradient of the blocked convolution: dbias (K * By * Bx floats, bias_mode 0 per block or
 // 1 shared) = the sum of dy over every output position of each block, in a fixed order, through
 // f32_block_dbias_workspace bytes of `ws` (nonzero for any non-empty dy).

@@ -117,3 +117,82 @@ def test_small_inputs(device, scale):
     want, = torch.autograd.grad(conv64(xg, wt, case[7]), xg, dy.double())
     mag, = torch.autograd.grad(conv64(xg, wt.abs(), case[7]), xg, dy.double().abs())
     check(dx.cpu(), want, mag, 9 * 36)
+
+
+# filter gradients: (n, h, w, c, k, r, s, conv); channel counts on both sides of the wave layouts
+GRADS = [
+    (2, 9, 11, 4, 8, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (3, 19, 17, 36, 68, 3, 3, (1, 1, 1, 1, 1, 1, 1)),     # channels past the tiles
+    (9, 7, 7, 64, 96, 3, 3, (1, 1, 1, 1, 1, 1, 1)),       # several images per tile
+    (2, 31, 29, 32, 32, 3, 3, (1, 1, 2, 2, 1, 1, 1)),     # stride, four wave groups
+    (1, 26, 40, 68, 28, 3, 3, (2, 0, 1, 2, 2, 1, 1)),     # dilation, two wave groups
+    (2, 21, 18, 20, 72, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (2, 15, 14, 128, 64, 1, 1, (0, 0, 1, 1, 1, 1, 1)),    # one tap, two channel tiles per wave
+    (2, 13, 15, 16, 40, 2, 3, (1, 1, 1, 1, 1, 1, 1)),     # fewer taps than a workgroup takes
+    (1, 20, 22, 64, 64, 5, 5, (2, 2, 1, 1, 1, 1, 1)),     # more
+    (2, 16, 16, 96, 64, 3, 3, (1, 1, 1, 1, 1, 1, 2)),     # groups
+    (1, 56, 56, 64, 64, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+]
+
+
+def grad_want(x, dy, wshape, conv, f=lambda v: v):
+    w = torch.zeros(wshape, dtype=torch.float64, requires_grad=True)
+    return torch.autograd.grad(conv64(f(x), w, conv), w, f(dy).double())[0]
+
+
+@pytest.mark.parametrize("case", GRADS, ids=[str(c) for c in GRADS])
+def test_filter_gradient(device, case):
+    n, h, w, c, k, r, s, conv = case
+    x, wt = data(case, 31 + GRADS.index(case))
+    dy = torch.randn(conv64(x, wt, conv).shape, generator=torch.Generator().manual_seed(4))
+    dw = torch.full(wt.shape, 7.0, device=device)
+    M.launch_grad_nhwc(x.to(device), dy.to(device), dw, n, h, w, c, r, s, k, conv)
+    # K-blocks of 32 positions, then the splits
+    check(dw.cpu(), grad_want(x, dy, wt.shape, conv), grad_want(x, dy, wt.shape, conv, torch.abs), dy[..., 0].numel() + 512)
+
+
+@pytest.mark.parametrize("grid", [(2, 3), (4, 1)])
+def test_blocked_filter_gradient(device, grid):
+    n, h, w, c, k = 5, 16, 18, 40, 70
+    by, bx = grid
+    gen = torch.Generator().manual_seed(8)
+    x, dy = torch.randn((n, h, w, c), generator=gen), torch.randn((n, h, w, k + 2), generator=gen)
+    k += 2
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    dw = torch.empty((k, by, bx, 3, 3, c), device=device)
+    M.launch_block_grad_nhwc(x.to(device), dy.to(device), dw, n, h, w, c, 3, 3, k,
+                             M.BlockConv2DParams(M.Conv2DParams(*conv), by, bx))
+    got = dw.cpu()
+    for i in range(by):
+        for j in range(bx):
+            d = torch.zeros_like(dy)
+            rows, cols = slice(i * h // by, (i + 1) * h // by), slice(j * w // bx, (j + 1) * w // bx)
+            d[:, rows, cols] = dy[:, rows, cols]
+            check(got[:, i, j], grad_want(x, d, (k, 3, 3, c), conv), grad_want(x, d, (k, 3, 3, c), conv, torch.abs), n * h * w)
+
+
+@pytest.mark.parametrize("shape", [(2, 24, 24, 64, 64), (2, 24, 24, 32, 32)])
+def test_filter_gradient_of_special_values(device, shape):
+    n, h, w, c, k = shape
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    gen = torch.Generator().manual_seed(9)
+    x, dy = torch.randn((n, h, w, c), generator=gen), torch.randn((n, h, w, k), generator=gen)
+    args = (n, h, w, c, 3, 3, k, conv)
+    dw = torch.empty((k, 3, 3, c), device=device)
+    M.launch_grad_nhwc((x * 2.0 ** -130).to(device), (dy * 2.0 ** 20).to(device), dw, *args)
+    xs, ds = x * 2.0 ** -130, dy * 2.0 ** 20
+    check(dw.cpu(), grad_want(xs, ds, (k, 3, 3, c), conv), grad_want(xs, ds, (k, 3, 3, c), conv, torch.abs), n * h * w + 512)
+    x[0, 5, 6, 3], x[1, 9, 9, 9] = float("inf"), float("nan")
+    M.launch_grad_nhwc(x.to(device), dy.to(device), dw, *args)
+    got = dw.cpu()
+    clean = torch.nan_to_num(x, nan=0.0, posinf=0.0)
+    want = grad_want(clean, dy, (k, 3, 3, c), conv)
+    for i in range(3):
+        for j in range(3):
+            want[:, i, j, 3] += float("inf") * dy[0, 5 - i + 1, 6 - j + 1].double()
+            want[:, i, j, 9] = float("nan")
+    assert torch.equal(got.isnan(), want.isnan())
+    fin = want.isfinite()
+    assert torch.equal(got[~fin & ~want.isnan()].double(), want[~fin & ~want.isnan()])
+    mag = grad_want(clean, dy, (k, 3, 3, c), conv, torch.abs)
+    assert bool(((got.double() - want).abs()[fin] <= (n * h * w) * 2.0 ** -23 * mag[fin]).all())

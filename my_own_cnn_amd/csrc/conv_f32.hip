@@ -20,7 +20,7 @@
 //     taps outside the image, values past kdim and rows past M or Kg read a valid address
 //     and are zeroed (or never stored), so the compiler's load counters stay exact.
 //   It serves what the split-bf16 kernel (conv_f32_split.hip) leaves to it: one-tap layers of a
-//   short reduction, few output channels at a stride, dilation below 1, the dx of a blocked filter.
+//   short reduction, few output channels at a stride, dilation below 1.
 //   The sum order differs from the reference's sequential fp32 loop; results agree within
 //   the reference's own check (verify_tensors with abs 1e-4 / rel 1e-3, main.cpp:306-316).
 //
@@ -1484,7 +1484,7 @@ hipError_t launch_f32_bprop_igemm(const Geom& g, const BlockGeom& bg, const floa
                                   hipStream_t stream) {
   const Geom b = f32_bprop_as_fprop(g);
   hipError_t e;
-  if (bg.By * bg.Bx == 1 && launch_f32_split(b, dense_blocks(b), dy, w, nullptr, 0, dx, true, stream, &e)) return e;
+  if (launch_f32_split(b, bg, dy, w, nullptr, 0, dx, true, stream, &e)) return e;
   return f32_igemm_launch(b, bg, bprop_regions(b, bg), dy, w, nullptr, 0, dx, true, stream);
 }
 

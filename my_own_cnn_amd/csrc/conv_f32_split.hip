@@ -42,6 +42,10 @@
 namespace miq {
 namespace {
 
+constexpr int kSplitMaxReach = 64;         // filter blocks that the halo of a tile touches (blocked dx)
+// floor(65536 / n) + 1: t / n = t * kInv16[n] >> 16 for t < 256
+__constant__ unsigned kInv16[17] = {0, 65537, 32769, 21846, 16385, 13108, 10923, 9363, 8193,
+                                    7282, 6554, 5958, 5462, 5042, 4682, 4370, 4097};
 constexpr int kSplitUnits = 4;             // halo (position, octet) pairs per thread
 constexpr int kSplitMaxOct = 1024;         // (tap, octet) pairs of a chunk
 
@@ -67,15 +71,33 @@ struct SplitArgs {
   int noct;        // R * S * co
   int nst;         // stages per chunk
   int ow_taps, ow_cg;  // transposed filter: R * S and channels per group of the original
-  int rx, nreg, rh, rw;  // output regions (the filter blocks) of rh x rw positions, rx per row
+  int rx, nreg, rh, rw;  // output regions of rh x rw positions, rx per row (forward: the filter blocks)
   int By, Bx, bias_mode;
-  FastDivM fd_tn, fd_tiles, fd_reg, fd_rx, fd_ntx, fd_nty, fd_co, fd_s, fd_hw, fd_hhw, fd_twp, fd_thw;
+  int bho, bwo;  // positions of a filter block (blocked dx: of dy)
+  int nfast;     // tile positions in (row, column, image) order instead of (image, row, column)
+  FastDivM fd_tn, fd_tiles, fd_reg, fd_rx, fd_ntx, fd_nty, fd_co, fd_s, fd_hw, fd_hhw, fd_twp, fd_thw, fd_ti;
 };
 
 __device__ __forceinline__ int f32s_slot(int row, int g) { return 4 * row + (g ^ (((row >> 3) & 1) << 1)); }
 
-template <bool TRANS, int NSEG, int WM, int WN>
+// MODE kSplitFwd: the forward convolution, a region's positions use its block's filter.  kSplitTrans:
+// the filter read as the dx filter of a stride-1 convolution (ow_* extents).  kSplitTransBlocked:
+// the same with a blocked filter, whose blocks partition this kernel's input (dy): a chunk's halo
+// is staged once and the reduction runs once per block that the tile's taps reach, over the taps
+// that reach it, each lane reading zeros for the positions of other blocks and each pair of
+// segments skipping the taps that none of its lanes uses.  With the image the fastest index of a
+// tile (16 images: a segment is one position) nearly every tap of a segment falls in one block.
+// Measured (us; before: the fp32 implicit GEMM's blocked form): 32 x 28 x 28, 128 -> 256 in 2 x 4
+// blocks 216 (366); 32 x 56 x 56, 64 -> 64 in 2 x 2 119 (123), in 4 x 4 117 (155); one image in
+// 4 x 4 38 (78). The stages of a neighbour's few taps bound it: a stage's filter values cost the
+// same whatever its MFMAs, so fetching them two stages ahead and keeping the reach in LDS (five
+// divisions a block otherwise) took the first from 404 to 226.
+enum SplitMode : int { kSplitFwd = 0, kSplitTrans = 1, kSplitTransBlocked = 2 };
+
+template <int MODE, int NSEG, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a) {
+  constexpr bool TRANS = MODE != kSplitFwd;
+  constexpr bool MULTI = MODE == kSplitTransBlocked;
   constexpr int NT = 64 * WM * WN;
   constexpr int BM = 16 * NSEG * WM;
   constexpr int BN = 32 * WN;
@@ -117,11 +139,19 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
 
   // a tile position m: image, row and column in the tile, and whether it is an output
   auto decode = [&](int m, int& im, int& lr, int& lc) -> bool {
-    im = fdiv(m, a.fd_thw);
-    const int p = m - im * (a.th * a.twp);
+    int p;
+    if (MULTI && a.nfast) {
+      p = fdiv(m, a.fd_ti);
+      im = m - p * a.ti;
+      if (p >= a.th * a.twp) return false;
+    } else {
+      im = fdiv(m, a.fd_thw);
+      p = m - im * (a.th * a.twp);
+    }
     lr = fdiv(p, a.fd_twp);
     lc = p - lr * a.twp;
-    return im < a.ti && img0 + im < g.N && lc < a.tw && ty0 + lr < a.rh && tx0 + lc < a.rw;
+    return im < a.ti && img0 + im < g.N && lc < a.tw && ty0 + lr < a.rh && tx0 + lc < a.rw &&
+           (!MULTI || (row0 + ty0 + lr < g.Ho && col0 + tx0 + lc < g.Wo));  // the last regions are clipped
   };
 
   // LDS slot (in units of 48 bytes) of octet oc's plane.  ds_read_b128 serves lane quads of both
@@ -162,7 +192,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   int boct[BU], bslot[BU];
   unsigned boff[BU];
   const int nblk = a.By * a.Bx;
-  const int ko_stride = a.ow_taps * a.ow_cg;
+  const int blk_stride = a.ow_taps * a.ow_cg;             // transposed: between filter blocks
+  const int ko_stride = MULTI ? blk_stride * nblk : blk_stride;  // and between original channels
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(
       TRANS ? a.w + static_cast<size_t>(grp) * g.Cg * ko_stride
             : a.w + (static_cast<size_t>(grp) * g.Kg * nblk + reg) * a.kdim, 0x7fffffff);
@@ -185,6 +216,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   }
   int* const flag = tab + a.nst * SO;
   if (t == 0) *flag = 0;
+  // MULTI: 48 bytes of zeros behind the table, at a 16-byte boundary
+  const int zoff = (static_cast<int>(reinterpret_cast<char*>(flag + 4) - reinterpret_cast<char*>(lds)) & ~15);
+  if (MULTI && t < 12) reinterpret_cast<int*>(reinterpret_cast<char*>(lds) + zoff)[t] = 0;
 
   // the tile's segments of 16 positions, spread evenly over the WM rows of waves: this wave's
   // first, how many are its own, and whether that is NSEG (else it computes NSEG - 1 and keeps its own)
@@ -203,7 +237,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   }
 
   v4f va[kSplitUnits][2];
-  v4f vb[BU][2];
+  v4f vb[MULTI ? 2 : 1][BU][2];  // filter values in flight, MULTI: of two stages
   unsigned mn = 0xffffffffu;
   const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
   auto load_a = [&](int c) {
@@ -226,33 +260,107 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   };
-  auto load_b = [&](int c, int s) {
+  // The filter blocks a tile reaches (MULTI; else one block with every tap): the taps r0.., s0.. of
+  // nr x ns that read the block and the block's rows and columns of the input.
+  struct Reach {
+    int idx, r0, s0, nr, ns, y0, y1, x0, x1, fblk, noct, nst;
+    unsigned inv;  // tap / ns = tap * inv >> 16 (tap < 256)
+  };
+  int bqx0 = 0, bnx = 1, bqy0 = 0, nreach = 1;
+  if constexpr (MULTI) {
+    const int ylo = max(h0, 0), yhi = min(h0 + a.hh, g.H) - 1, xlo = max(w0, 0), xhi = min(w0 + a.hw, g.W) - 1;
+    nreach = 0;
+    if (ylo <= yhi && xlo <= xhi) {
+      bqy0 = ylo / a.bho;
+      bqx0 = xlo / a.bwo;
+      bnx = xhi / a.bwo - bqx0 + 1;
+      nreach = (yhi / a.bho - bqy0 + 1) * bnx;
+    }
+  }
+  // MULTI: the reach's blocks, 8 ints each behind the zeros: r0 | nr << 8 | s0 << 16 | ns << 24 (0: no
+  // tap reads the block), rows y0, y1, columns x0, x1, element offset of the block's filter
+  int* const rtab = reinterpret_cast<int*>(reinterpret_cast<char*>(lds) + zoff + 48);
+  if constexpr (MULTI) {
+    if (t < nreach) {
+      const int qy = t / bnx, qx = t - qy * bnx;
+      const int y0 = (bqy0 + qy) * a.bho, x0 = (bqx0 + qx) * a.bwo;
+      const int y1 = min(y0 + a.bho, g.H) - 1, x1 = min(x0 + a.bwo, g.W) - 1;
+      const int ra = y0 - h0 - (a.th - 1), sa = x0 - w0 - (a.tw - 1);
+      const int r0 = ra > 0 ? (ra + g.dh - 1) / g.dh : 0, s0 = sa > 0 ? (sa + g.dw - 1) / g.dw : 0;
+      const int nr = y1 >= h0 ? min(g.R - 1, (y1 - h0) / g.dh) - r0 + 1 : 0;
+      const int ns = x1 >= w0 ? min(g.S - 1, (x1 - w0) / g.dw) - s0 + 1 : 0;
+      rtab[8 * t] = nr > 0 && ns > 0 ? r0 | nr << 8 | s0 << 16 | ns << 24 : 0;
+      rtab[8 * t + 1] = y0;
+      rtab[8 * t + 2] = y1;
+      rtab[8 * t + 3] = x0;
+      rtab[8 * t + 4] = x1;
+      rtab[8 * t + 5] = ((bqy0 + qy) * a.Bx + bqx0 + qx) * blk_stride;
+    }
+    __syncthreads();
+  }
+  // block `idx` of the reach or the next one with taps; idx == nreach: none left
+  auto set_reach = [&](Reach& b, int idx) {
+    b.idx = idx;
+    if constexpr (!MULTI) {
+      b.noct = a.noct;
+      b.nst = a.nst;
+    } else {
+      int packed = 0;
+      for (; b.idx < nreach; ++b.idx) {
+        packed = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx]);
+        if (packed != 0) break;
+      }
+      if (b.idx < nreach) {
+        b.r0 = packed & 0xff;
+        b.nr = (packed >> 8) & 0xff;
+        b.s0 = (packed >> 16) & 0xff;
+        b.ns = packed >> 24;
+        b.y0 = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx + 1]);
+        b.y1 = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx + 2]);
+        b.x0 = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx + 3]);
+        b.x1 = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx + 4]);
+        b.fblk = __builtin_amdgcn_readfirstlane(rtab[8 * b.idx + 5]);
+        b.noct = b.nr * b.ns * a.co;
+        b.nst = (b.noct + SO - 1) / SO;
+        b.inv = kInv16[b.ns];
+      }
+    }
+  };
+  auto load_b = [&](auto set, int c, int s, const Reach& rb) {
+    constexpr int V = MULTI ? decltype(set)::value : 0;
     const int c0 = 8 * a.co * c;
 #pragma unroll
     for (int j = 0; j < BU; ++j) {
       const int o = SO * s + boct[j];
       const int tap = fdiv(o, a.fd_co);
       const int ch = c0 + 8 * (o - tap * a.co);
-      const int left = o < a.noct ? g.Cg - ch : 0;
+      const int left = o < rb.noct ? g.Cg - ch : 0;
       if constexpr (TRANS) {
-        const unsigned off = boff[j] + 4u * (ch * ko_stride + (a.ow_taps - 1 - tap) * a.ow_cg);
+        int ft = tap, fblk = 0;
+        if constexpr (MULTI) {
+          const int tr = static_cast<int>((static_cast<unsigned>(tap) * rb.inv) >> 16);
+          ft = (rb.r0 + tr) * g.S + rb.s0 + tap - tr * rb.ns;
+          fblk = rb.fblk;
+        }
+        const unsigned off = boff[j] + 4u * (ch * ko_stride + fblk + (a.ow_taps - 1 - ft) * a.ow_cg);
         const unsigned o0 = left >= 4 ? off : kNone, o1 = left >= 8 ? off : kNone;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          vb[j][0][e] = buffer_load4(rw, o0, 4 * e * ko_stride);
-          vb[j][1][e] = buffer_load4(rw, o1, 4 * (e + 4) * ko_stride);
+          vb[V][j][0][e] = buffer_load4(rw, o0, 4 * e * ko_stride);
+          vb[V][j][1][e] = buffer_load4(rw, o1, 4 * (e + 4) * ko_stride);
         }
       } else {
         const unsigned off = boff[j] + 4u * (tap * g.Cg + ch);
-        vb[j][0] = buffer_load16(rw, left >= 4 ? off : kNone, 0);
-        vb[j][1] = buffer_load16(rw, left >= 8 ? off + 16u : kNone, 0);
+        vb[V][j][0] = buffer_load16(rw, left >= 4 ? off : kNone, 0);
+        vb[V][j][1] = buffer_load16(rw, left >= 8 ? off + 16u : kNone, 0);
       }
     }
   };
-  auto store_b = [&](int buf) {  // the values of the last load_b
+  auto store_b = [&](auto set, int buf) {  // the values of the set's last load_b
+    constexpr int V = MULTI ? decltype(set)::value : 0;
 #pragma unroll
     for (int j = 0; j < BU; ++j) {
-      const Split8 sp = split8(vb[j][0], vb[j][1], mn);
+      const Split8 sp = split8(vb[V][j][0], vb[V][j][1], mn);
 #pragma unroll
       for (int p = 0; p < 3; ++p) sB[buf * BSZ + bslot[j] + p] = sp.p[p];
     }
@@ -271,11 +379,24 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   // steps of up to two segments; a step's fragments are read while the step before it computes.
   // The six products of a step sum from zero, smallest first, and are added to the accumulators.
   int lc = 0, ls = 0;  // stage of the next load_b
-  auto fetch = [&]() {
-    load_b(lc, ls);
-    if (++ls == a.nst) {
+  Reach lb;
+  set_reach(lb, 0);
+  const int first_reach = lb.idx;
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  auto fetch = [&](auto set) {
+    load_b(set, lc, ls, lb);
+    if (++ls == lb.nst) {
       ls = 0;
-      lc = min(lc + 1, a.nchunk - 1);  // past the end: loaded, never used
+      if constexpr (MULTI) {
+        set_reach(lb, lb.idx + 1);
+        if (lb.idx >= nreach) {
+          set_reach(lb, 0);
+          lc = min(lc + 1, a.nchunk - 1);
+        }
+      } else {
+        lc = min(lc + 1, a.nchunk - 1);  // past the end: loaded, never used
+      }
     }
   };
   auto run = [&](auto ns) {
@@ -327,8 +448,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
               }
           }
           if constexpr (st == 0) {
-            store_b(buf ^ 1);
-            fetch();
+            store_b(even, buf ^ 1);
+            fetch(even);
             if (s == 0) load_a(more ? c + 1 : c);
           }
 #pragma unroll
@@ -356,15 +477,119 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   };
-  fetch();
-  load_a(0);
-  store_b(0);
-  fetch();
-  store_a();
-  __syncthreads();
-  // both arms run the same barriers
-  if (whole) run(std::integral_constant<int, NSEG>{});
-  else run(std::integral_constant<int, NSEG - 1>{});
+  // MULTI: the chunk's stages block after block, a K-block's fragments read where it is computed
+  auto run_blocks = [&]() {
+    int prow[NSEG], pcol[NSEG];  // this lane's positions on the input grid, tap (0, 0)
+#pragma unroll
+    for (int i = 0; i < NSEG; ++i) {
+      int im, lr, lcc;
+      const bool ok = i < own && decode(m0 + 16 * i, im, lr, lcc);
+      prow[i] = ok ? h0 + lr : INT32_MIN / 2;
+      pcol[i] = w0 + lcc;
+    }
+    Reach rb;
+    unsigned use[NSEG];  // rows r (bit r) and columns s (bit 16 + s) of the block
+    auto enter = [&](int idx) {
+      set_reach(rb, idx);
+      if (rb.idx >= nreach) return;
+#pragma unroll
+      for (int i = 0; i < NSEG; ++i) use[i] = 0;
+      for (int r = rb.r0; r < rb.r0 + rb.nr; ++r)
+#pragma unroll
+        for (int i = 0; i < NSEG; ++i)
+          use[i] |= static_cast<unsigned>(prow[i] + r * g.dh >= rb.y0 && prow[i] + r * g.dh <= rb.y1) << r;
+      for (int s = rb.s0; s < rb.s0 + rb.ns; ++s)
+#pragma unroll
+        for (int i = 0; i < NSEG; ++i)
+          use[i] |= static_cast<unsigned>(pcol[i] + s * g.dw >= rb.x0 && pcol[i] + s * g.dw <= rb.x1) << (16 + s);
+    };
+    // stage s of the block: the filter buffer and register set of its parity over all stages
+    auto stage = [&](auto par, auto other, int c, int s) {
+      constexpr int PAR = decltype(par)::value;
+      store_b(other, PAR ^ 1);
+      fetch(other);
+      if (s == 0 && rb.idx == first_reach) load_a(min(c + 1, a.nchunk - 1));
+#pragma unroll
+      for (int kb = 0; kb < SO / 4; ++kb) {
+        const int o = SO * s + 4 * kb + q;
+        if (SO * s + 4 * kb < rb.noct) {  // uniform
+          const int tap = fdiv(o, a.fd_co);
+          const int tr = static_cast<int>((static_cast<unsigned>(tap) * rb.inv) >> 16);
+          const int r = rb.r0 + tr, ss = rb.s0 + tap - tr * rb.ns;
+          const int ao = 48 * (plane(o - tap * a.co) + r * g.dh * a.hw + ss * g.dw);
+          const bool in = o < rb.noct;
+          v8b fb[2][3];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+              fb[j][p] = *reinterpret_cast<const v8b*>(bB + 16 * (PAR * BSZ + p) + 48 * (4 * kb * BN + 2 * kb * BSH + 16 * j));
+#pragma unroll
+          for (int i0 = 0; i0 < NSEG; i0 += 2) {
+            bool hit[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) hit[i] = in && ((use[i0 + i] >> r) & (use[i0 + i] >> (16 + ss)) & 1u) != 0;
+            if (__any(hit[0] || hit[1])) {
+              v8b fa[2][3];
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                const int ad = hit[i] ? pbase[i0 + i] + ao : zoff;
+#pragma unroll
+                for (int p = 0; p < 3; ++p) fa[i][p] = *reinterpret_cast<const v8b*>(bA + ad + 16 * p);
+              }
+              v4f z[2][2];
+#pragma unroll
+              for (int k = 0; k < 6; ++k) {
+                constexpr int kw[6] = {2, 0, 1, 1, 0, 0}, kx[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                  for (int j = 0; j < 2; ++j)
+                    z[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][kw[k]], fa[i][kx[k]], k == 0 ? zero : z[j][i], 0, 0, 0);
+              }
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[j][i0 + i] += z[j][i];
+            }
+          }
+        }
+      }
+      __syncthreads();
+    };
+    int c = 0, s = 0;
+    enter(0);
+    auto next = [&]() {  // the next stage: of the block, the next block, the next chunk
+      if (++s < rb.nst) return true;
+      s = 0;
+      enter(rb.idx + 1);
+      if (rb.idx < nreach) return true;
+      if (++c == a.nchunk) return false;
+      enter(0);
+      store_a();
+      __syncthreads();
+      return true;
+    };
+    while (true) {
+      stage(even, odd, c, s);
+      if (!next()) break;
+      stage(odd, even, c, s);
+      if (!next()) break;
+    }
+  };
+  // both arms run the same barriers; a tile that reaches no block is zero
+  if (!MULTI || first_reach < nreach) {
+    fetch(even);
+    load_a(0);
+    if constexpr (MULTI) fetch(odd);
+    store_b(even, 0);
+    fetch(even);
+    store_a();
+    __syncthreads();
+    if constexpr (MULTI) run_blocks();
+    else if (whole) run(std::integral_constant<int, NSEG>{});
+    else run(std::integral_constant<int, NSEG - 1>{});
+  }
 
   bool bad = mn < kSmall2;
 #pragma unroll
@@ -399,16 +624,22 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int i = 0; i < NSEG; ++i) acc[j][i] = zero;
-    for (int tap = 0; tap < g.R * g.S; ++tap) {
+    for (int tb = 0; tb < g.R * g.S * (MULTI ? nreach : 1); ++tb) {  // taps, MULTI: of each block
+      const int bi = MULTI ? tb / (g.R * g.S) : 0;
+      const int tap = tb - bi * (g.R * g.S);
       const int r = fdiv(tap, a.fd_s);
       const int s = tap - r * g.S;
+      const int qy = bqy0 + bi / bnx, qx = bqx0 + bi - bi / bnx * bnx;
+      const int ylo = MULTI ? qy * a.bho : 0, yhi = MULTI ? min(ylo + a.bho, g.H) : g.H;
+      const int xlo = MULTI ? qx * a.bwo : 0, xhi = MULTI ? min(xlo + a.bwo, g.W) : g.W;
+      const size_t fblk = MULTI ? static_cast<size_t>(qy * a.Bx + qx) * blk_stride : 0;
       for (int c0 = 0; c0 < g.Cg; c0 += 16) {
         __syncthreads();  // the previous step's reads (and the flag's)
         const int ch = c0 + 4 * (t & 3);
 #pragma unroll
         for (int k = 0; k < UR; ++k) {
           const int hi = uh[k] + r * g.dh, wi = uw[k] + s * g.dw;
-          const bool ok = ch < g.Cg && hi >= 0 && hi < g.H && wi >= 0 && wi < g.W;
+          const bool ok = ch < g.Cg && hi >= ylo && hi < yhi && wi >= xlo && wi < xhi;
           const v4f v = *reinterpret_cast<const v4f*>(ok ? ux[k] + (static_cast<size_t>(hi) * g.W + wi) * g.C + ch : a.x);
           fA[f32s_slot((t + NT * k) >> 2, t & 3)] = ok ? v : zero;
         }
@@ -419,7 +650,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
           if (cb < g.Cg) {
             if constexpr (TRANS) {
               const float* p = a.w + (static_cast<size_t>(grp) * g.Cg + cb) * ko_stride +
-                               static_cast<size_t>(a.ow_taps - 1 - tap) * a.ow_cg + kr;
+                               fblk + static_cast<size_t>(a.ow_taps - 1 - tap) * a.ow_cg + kr;
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] = p[e * ko_stride];
             } else {
@@ -497,7 +728,7 @@ constexpr SplitVariant kVariants[] = {{4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {4, 4, 1}
 // Estimated cycles of a launch: rounds of workgroups over the 256 CUs x (K-blocks at the MFMA rate
 // of a wave's tile, the staged values, a fixed start and end).
 void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int th, int tw, int twp,
-              SplitPlan* best) {
+              bool blocked_dx, SplitPlan* best) {
   const SplitVariant& V = kVariants[v];
   const int nt = 64 * V.wm * V.wn, bn = 32 * V.wn, so = std::max(4, 2 * V.wm);
   SplitPlan p{};
@@ -531,13 +762,23 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
     p.hps = (p.hp + 15) & ~15;
     p.ash = co >= 6 ? 2 : (co >= 4 ? 4 : 0);
     const int bsz = 3 * (so * bn + (16 / so) * so / 2);
-    p.lds = static_cast<size_t>(3 * (co * p.hps + 8) + 2 * bsz) * 16 + static_cast<size_t>(p.nst * so + 1) * 4;
+    p.lds = static_cast<size_t>(3 * (co * p.hps + 8) + 2 * bsz) * 16 + static_cast<size_t>(p.nst * so + 1) * 4 +
+            (blocked_dx ? 80 + 32 * kSplitMaxReach : 0);
     if (p.lds > kSplitLds) continue;
     const int per_cu = std::max(1, std::min<int>({static_cast<int>(kSplitLds / p.lds), 8 / (V.wm * V.wn), 4}));
     const double kb = static_cast<double>(p.nchunk) * ((p.noct + 3) / 4);
     const double mfma = kb * V.nseg * 12 * 16.0 * V.wm * V.wn / 4;  // SIMD cycles of a workgroup
     const double stage = p.nchunk * (static_cast<double>(p.hp) * co + static_cast<double>(p.nst) * so * bn) * 60.0 / 64;
-    const double wg = mfma * 1.25 + stage * 0.7 + 2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
+    double wg = mfma * 1.25 + stage * 0.7 + 2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
+    if (blocked_dx) {
+      // a tile edge on a block edge adds the taps that cross it: (block, tap) pairs and blocks of
+      // an average tile; a stage takes at least its filter values' way through the registers
+      const double pairs = (g.R + (g.R - 1.0) / p.nty) * (g.S + (g.S - 1.0) / p.ntx);
+      const double blks = (1 + (g.R > 1 ? 2.0 : 0.0) / p.nty) * (1 + (g.S > 1 ? 2.0 : 0.0) / p.ntx);
+      const double stages = p.nchunk * (pairs * co / so + 0.5 * blks);
+      wg = std::max(mfma * 1.25, stages * 2200.0) + 0.3 * std::min(mfma, stages * 2200.0) + stage * 0.7 +
+           2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
+    }
     const double rounds = std::ceil(static_cast<double>(p.blocks) / (256.0 * per_cu)) * per_cu;
     p.cost = std::min(rounds, static_cast<double>(p.blocks) / 256.0 + 0.5 * per_cu) * wg;
     if (p.blocks < 256) p.cost = wg;
@@ -575,34 +816,70 @@ SplitPlan make_plan(const Geom& g, int rh, int rw, long long nreg, bool transpos
       th = (rh + (rh + th - 1) / th - 1) / ((rh + th - 1) / th);  // even rows of tiles
       const int ti = th == rh && tw == rw ? std::max(1, std::min(g.N, bm / (th * tw))) : 1;
       const int tw16 = (tw + 15) & ~15;  // rows of whole segments: no segment wraps into the next row
-      if (tw16 != tw && ti * th * tw16 <= bm) consider(g, rh, rw, nreg, v, ti, th, tw, tw16, &best);
-      else consider(g, rh, rw, nreg, v, ti, th, tw, tw, &best);
+      if (tw16 != tw && ti * th * tw16 <= bm) consider(g, rh, rw, nreg, v, ti, th, tw, tw16, false, &best);
+      else consider(g, rh, rw, nreg, v, ti, th, tw, tw, false, &best);
       if (tw <= 8) break;
     }
   }
   return best;
 }
 
-template <bool TRANS, int NSEG, int WM, int WN>
+template <int MODE, int NSEG, int WM, int WN>
 hipError_t launch_variant(const SplitArgs& a, const SplitPlan& p, hipStream_t stream) {
   if (p.lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&f32_split_kernel<TRANS, NSEG, WM, WN>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&f32_split_kernel<MODE, NSEG, WM, WN>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kSplitLds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((f32_split_kernel<TRANS, NSEG, WM, WN>), dim3(static_cast<unsigned>(p.blocks)),
+  hipLaunchKernelGGL((f32_split_kernel<MODE, NSEG, WM, WN>), dim3(static_cast<unsigned>(p.blocks)),
                      dim3(64 * WM * WN), p.lds, stream, a);
   return hipGetLastError();
 }
 
-template <bool TRANS>
+template <int MODE>
 hipError_t launch_split(const SplitArgs& a, const SplitPlan& p, hipStream_t stream) {
   switch (p.variant) {
-    case 0: return launch_variant<TRANS, 4, 4, 2>(a, p, stream);
-    case 1: return launch_variant<TRANS, 4, 2, 2>(a, p, stream);
-    case 2: return launch_variant<TRANS, 2, 2, 2>(a, p, stream);
-    default: return launch_variant<TRANS, 4, 4, 1>(a, p, stream);
+    case 0: return launch_variant<MODE, 4, 4, 2>(a, p, stream);
+    case 1: return launch_variant<MODE, 4, 2, 2>(a, p, stream);
+    case 2: return launch_variant<MODE, 2, 2, 2>(a, p, stream);
+    default: return launch_variant<MODE, 4, 4, 1>(a, p, stream);
   }
+}
+
+}  // namespace
+
+namespace {
+
+// Blocked dx: 16 images (or all of fewer) x a few positions per tile, tiles inside regions of
+// ceil(Ho / By) x ceil(Wo / Bx), so that most reach one filter block.
+SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) {
+  SplitPlan best{};
+  best.variant = -1;
+  const long long nreg = static_cast<long long>(bg.By) * bg.Bx;
+  if (g.dh <= 0 || g.dw <= 0 || g.R > 16 || g.S > 16) return best;
+  if (g.R * g.S == 1 && g.Cg < 128) return best;
+  if (static_cast<double>(g.Kg) * nreg * g.R * g.S * g.Cg * 4 >= 2147483647.0) return best;
+  for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
+    if ((kVariants[v].wn == 1) != (g.Kg <= 32)) continue;
+    const int bm = 16 * kVariants[v].nseg * kVariants[v].wm;
+    for (const int images : {16, 8, 4, 2, 1}) {
+      if (images > g.N && images != 1) continue;
+      const int pos = bm / images;
+      int last = 0;
+      for (int j = 1; j <= 16; ++j) {
+        const int tw = (rw + j - 1) / j;
+        if (tw > pos || tw == last) continue;
+        last = tw;
+        int th = std::min(rh, pos / tw);
+        th = (rh + (rh + th - 1) / th - 1) / ((rh + th - 1) / th);
+        const int hh = th + (g.R - 1) * g.dh, hw = tw + (g.S - 1) * g.dw;
+        if ((hh / bg.bho + 2) * (hw / bg.bwo + 2) > kSplitMaxReach) continue;
+        consider(g, rh, rw, nreg, v, images, th, tw, tw, true, &best);
+        if (tw <= 2) break;
+      }
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -610,7 +887,11 @@ hipError_t launch_split(const SplitArgs& a, const SplitPlan& p, hipStream_t stre
 bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                       int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err) {
   const int nreg = bg.By * bg.Bx;
-  const SplitPlan p = make_plan(g, bg.bho, bg.bwo, nreg, transposed);
+  const bool blocked_dx = transposed && nreg > 1;
+  // the output regions: forward the filter blocks; blocked dx as many of the dx grid
+  const int rh = blocked_dx ? (g.Ho + bg.By - 1) / bg.By : (transposed ? g.Ho : bg.bho);
+  const int rw = blocked_dx ? (g.Wo + bg.Bx - 1) / bg.Bx : (transposed ? g.Wo : bg.bwo);
+  const SplitPlan p = blocked_dx ? make_blocked_plan(g, bg, rh, rw) : make_plan(g, rh, rw, nreg, transposed);
   if (p.variant < 0 || p.blocks <= 0 || p.blocks > (1LL << 22)) return false;
   SplitArgs a;
   a.x = x; a.w = w; a.bias = bias; a.y = y; a.g = g;
@@ -623,7 +904,8 @@ bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const 
   a.co = p.co; a.nchunk = p.nchunk; a.noct = p.noct; a.nst = p.nst;
   a.ow_taps = g.R * g.S;
   a.ow_cg = g.Kg;
-  a.rx = bg.Bx; a.nreg = nreg; a.rh = bg.bho; a.rw = bg.bwo;
+  a.rx = bg.Bx; a.nreg = nreg; a.rh = rh; a.rw = rw;
+  a.bho = bg.bho; a.bwo = bg.bwo; a.nfast = blocked_dx ? 1 : 0;
   a.By = bg.By; a.Bx = bg.Bx; a.bias_mode = bias_mode;
   a.fd_tn = fastdiv_m(a.tn);
   a.fd_tiles = fastdiv_m(a.tiles);
@@ -637,7 +919,10 @@ bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const 
   a.fd_hhw = fastdiv_m(a.hh * a.hw);
   a.fd_twp = fastdiv_m(a.twp);
   a.fd_thw = fastdiv_m(a.th * a.twp);
-  *err = transposed ? launch_split<true>(a, p, stream) : launch_split<false>(a, p, stream);
+  a.fd_ti = fastdiv_m(a.ti);
+  *err = blocked_dx   ? launch_split<kSplitTransBlocked>(a, p, stream)
+         : transposed ? launch_split<kSplitTrans>(a, p, stream)
+                      : launch_split<kSplitFwd>(a, p, stream);
   return true;
 }
 

@@ -199,8 +199,8 @@ bool f32_igemm_eligible(const Geom& g, const BlockGeom& bg, const void* x, const
 hipError_t launch_f32_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                             int bias_mode, float* y, hipStream_t stream);
 // The same forward pass on the bf16 matrix cores, each operand split into three bf16 numbers
-// (fp32 accuracy); `transposed`: the dx of a stride-1 convolution with a plain filter, g and bg
-// those of f32_bprop_as_fprop.  False when no tile of the shape fits (nothing is launched).
+// (fp32 accuracy); `transposed`: the dx of a stride-1 convolution, g of f32_bprop_as_fprop and bg
+// the blocks of the original output.  False when no tile of the shape fits (nothing is launched).
 bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                       int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err);
 hipError_t launch_f32_direct(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,

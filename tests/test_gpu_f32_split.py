@@ -83,6 +83,52 @@ def test_blocked_forward(device, grid):
             check(y[:, rows, cols].cpu(), conv64(x, f, conv)[:, rows, cols], conv64(x.abs(), f.abs(), conv)[:, rows, cols], 9 * c)
 
 
+def blocked_dx(dy, wt, xshape, conv):
+    """dx of a blocked convolution and the sum of its terms' magnitudes, in 64 bits."""
+    by, bx = wt.shape[1:3]
+    h, w = dy.shape[1:3]
+    x = torch.zeros(xshape, dtype=torch.float64, requires_grad=True)
+    out = [0, 0]
+    for i in range(by):
+        for j in range(bx):
+            d = torch.zeros_like(dy)
+            rows, cols = slice(i * h // by, (i + 1) * h // by), slice(j * w // bx, (j + 1) * w // bx)
+            d[:, rows, cols] = dy[:, rows, cols]
+            f = wt[:, i, j].contiguous()
+            for a, fn in enumerate((lambda v: v, torch.abs)):
+                out[a] = out[a] + torch.autograd.grad(conv64(x, fn(f), conv), x, fn(d).double())[0]
+    return out
+
+
+# (n, h, w, c, k, r, s, conv, by, bx): images above and below a segment's 16, blocks of a few
+# positions, taps that reach past a neighbour block, clipped regions, groups, 32 channels a group
+BLOCKED_DX = [
+    (3, 16, 18, 40, 72, 3, 3, (1, 1, 1, 1, 1, 1, 1), 2, 3),
+    (20, 12, 14, 36, 24, 3, 3, (1, 1, 1, 1, 1, 1, 1), 4, 2),
+    (17, 12, 12, 24, 16, 5, 5, (2, 2, 1, 1, 1, 1, 1), 6, 4),
+    (2, 14, 15, 48, 40, 3, 3, (2, 0, 1, 1, 2, 1, 1), 2, 1),
+    (16, 10, 9, 64, 128, 3, 2, (0, 1, 1, 1, 1, 1, 2), 4, 2),
+    (33, 8, 8, 40, 160, 1, 1, (0, 0, 1, 1, 1, 1, 1), 2, 2),
+]
+
+
+@pytest.mark.parametrize("case", BLOCKED_DX, ids=str)
+def test_blocked_dx(device, case):
+    n, h, w, c, k, r, s, conv, by, bx = case
+    gen = torch.Generator().manual_seed(12)
+    p = M.BlockConv2DParams(M.Conv2DParams(*conv), by, bx)
+    ho, wo = M.infer_block_conv_shape(n, h, w, c, r, s, k, p)[:2]
+    wt = torch.randn((k, by, bx, r, s, c // conv[6]), generator=gen)
+    dy = torch.randn((n, ho, wo, k), generator=gen)
+    dx = torch.full((n, h, w, c), 7.0, device=device)
+    for special in (False, True):
+        if special:  # one value sends its tiles through the fp32 instructions
+            dy[0, ho // 2, wo // 2, 1] = 2.0 ** -130
+        M.launch_block_bprop_nhwc(dy.to(device), wt.to(device), dx, n, h, w, c, r, s, k, p)
+        want, mag = blocked_dx(dy, wt, (n, h, w, c), conv)
+        check(dx.cpu(), want, mag, r * s * k // conv[6])
+
+
 def test_infinite_and_nan_inputs(device):
     x, wt = data((2, 20, 20, 32, 40, 3, 3, (1, 1, 1, 1, 1, 1, 1)), 5)
     x[0, 3, 4, 5], x[0, 10, 12, 7], x[1, 19, 19, 31], x[1, 0, 0, 0] = float("inf"), float("nan"), float("-inf"), 3.4e38

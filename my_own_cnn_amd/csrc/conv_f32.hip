@@ -768,6 +768,124 @@ __global__ void __launch_bounds__(kDirectThreads) f32_bprop_direct4_kernel(const
   store_gap(acc);
 }
 
+// The same dx, bit for bit, with 4 channels x kTilePix pixels per thread (plain filter,
+// (C/groups) % 4 == 0, (K/groups) % 4 == 0, dy, w and dx 16-byte aligned).  The pixels of a thread
+// are a stride apart in one row, so the same taps reach them and a filter float4 serves all of
+// them; a workgroup's pixels share both phases (row and column modulo the stride), so its waves
+// run the same taps.  Per tap the workgroup copies the filter slice of its 4 QB channels, kTileKo
+// output channels at a time, to LDS; dy is read as float4s of 4 output channels.  Per 4 output
+// channels a thread issues 8 loads for 128 multiplies and adds; the one-pixel kernel above issues
+// 8 for 32 and is bound by them: 32 x 112 x 112 stride 2, 32 -> 32 281 -> 61 us; 8 x 56 x 56,
+// 128 -> 128 347 -> 71; 8 x 224 x 224 7x7, 4 -> 64 1417 -> 780.  Bound by the vector ALU now: one
+// multiply and one add per term, not contracted, are 51 us of the first at 2.2 GHz.
+constexpr int kTilePix = 4;
+constexpr int kTileKo = 128;
+
+struct TileDxArgs {
+  const float* dy;
+  const float* w;
+  float* dx;
+  Geom g;
+  int rows, cgs;  // rows and pixel groups per row of the largest phase
+  FastDivM fd_rows, fd_cgs, fd_sw;
+  long long groups;  // N * rows * cgs
+};
+
+template <int QB>
+__global__ void __launch_bounds__(kDirectThreads) f32_bprop_tile_kernel(TileDxArgs a) {
+  constexpr int P = kTilePix;
+  __shared__ v4f wl[kTileKo * QB];
+  const Geom& g = a.g;
+  const int t = threadIdx.x;
+  const int quad = t % QB;
+  const int phh = fdiv(blockIdx.y, a.fd_sw), phw = blockIdx.y - phh * g.sw;
+  const int c = 4 * (blockIdx.z * QB + quad);
+  const int grp = (4 * static_cast<int>(blockIdx.z) * QB) / g.Cg;  // 4 QB divides C/groups
+  const long long pg = static_cast<long long>(blockIdx.x) * (kDirectThreads / QB) + t / QB;
+  const int pgi = static_cast<int>(min(pg, a.groups - 1));
+  const int rem = fdiv(pgi, a.fd_cgs);
+  const int cg = pgi - rem * a.cgs;
+  const int n = fdiv(rem, a.fd_rows);
+  const int hi = phh + g.sh * (rem - n * a.rows);
+  const int w0 = phw + g.sw * P * cg;  // the thread's pixels: w0 + sw j
+  const bool live = pg < a.groups && hi < g.H && w0 < g.W;
+  const int kdim = g.R * g.S * g.Cg;
+  const float* const wg = a.w + static_cast<size_t>(grp) * g.Kg * kdim + (4 * static_cast<int>(blockIdx.z) * QB - grp * g.Cg);
+  v4f acc[P];
+#pragma unroll
+  for (int j = 0; j < P; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < g.R; ++r) {
+    if ((phh + g.ph - r * g.dh) % g.sh != 0) continue;  // uniform
+    const int hn = hi + g.ph - r * g.dh;
+    const int ho = hn / g.sh;
+    const bool rok = live && hn >= 0 && ho < g.Ho;
+    for (int s = 0; s < g.S; ++s) {
+      if ((phw + g.pw - s * g.dw) % g.sw != 0) continue;  // uniform
+      const int wo0 = (phw + g.pw - s * g.dw) / g.sw + P * cg;  // exact
+      bool ok[P];
+      bool all = true, any = false;
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        ok[j] = rok && w0 + g.sw * j < g.W && wo0 + j >= 0 && wo0 + j < g.Wo;
+        all = all && ok[j];
+        any = any || ok[j];
+      }
+      const float* dp[P];
+#pragma unroll
+      for (int j = 0; j < P; ++j)
+        dp[j] = a.dy + (ok[j] ? ((static_cast<size_t>(n) * g.Ho + ho) * g.Wo + wo0 + j) * g.K : 0) +
+                static_cast<size_t>(grp) * g.Kg;
+      const float* const wt = wg + static_cast<size_t>(r * g.S + s) * g.Cg;
+      for (int k0 = 0; k0 < g.Kg; k0 += kTileKo) {
+        const int kn = min(kTileKo, g.Kg - k0);
+        __syncthreads();  // the previous slice's reads
+        for (int u = t; u < kn * QB; u += kDirectThreads)
+          wl[u] = *reinterpret_cast<const v4f*>(wt + static_cast<size_t>(k0 + u / QB) * kdim + 4 * (u % QB));
+        __syncthreads();
+        if (__all(all)) {
+          for (int k = 0; k < kn; k += 4) {
+            v4f d[P], wv[4];
+#pragma unroll
+            for (int j = 0; j < P; ++j) d[j] = *reinterpret_cast<const v4f*>(dp[j] + k0 + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wv[e] = wl[(k + e) * QB + quad];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int j = 0; j < P; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[j][i] = __fadd_rn(acc[j][i], __fmul_rn(d[j][e], wv[e][i]));
+          }
+        } else if (__any(any)) {  // some pixels have no output position at this tap: their sums stay
+          for (int k = 0; k < kn; k += 4) {
+            v4f d[P], wv[4];
+#pragma unroll
+            for (int j = 0; j < P; ++j) d[j] = *reinterpret_cast<const v4f*>(dp[j] + k0 + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wv[e] = wl[(k + e) * QB + quad];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int j = 0; j < P; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  const float v = __fadd_rn(acc[j][i], __fmul_rn(d[j][e], wv[e][i]));
+                  acc[j][i] = ok[j] ? v : acc[j][i];
+                }
+          }
+        }
+      }
+    }
+  }
+  if (!live) return;  // after the last barrier
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+    if (w0 + g.sw * j < g.W) {
+      *reinterpret_cast<v4f*>(a.dx + ((static_cast<size_t>(n) * g.H + hi) * g.W + w0 + g.sw * j) * g.C + c) = acc[j];
+      store_gap(acc[j]);
+    }
+}
+
 // Depthwise dx (C/groups == K/groups == 1, C % 4 == 0, plain filter): one thread per input
 // pixel and 4 consecutive channels, the filter staged in LDS as [tap][channel] as in
 // f32_depthwise_kernel, one float4 of dy per tap.  Channel c's sum runs over the taps (r, s)
@@ -1319,8 +1437,42 @@ hipError_t launch_f32_depthwise_bprop(const Geom& g, const float* dy, const floa
   return hipGetLastError();
 }
 
+namespace {
+
+// False where the tiled kernel does not take the problem.
+bool launch_bprop_tile(const Geom& g, const BlockGeom& bg, const float* dy, const float* w, float* dx,
+                       hipStream_t stream) {
+  if (bg.By * bg.Bx != 1 || g.Cg % 4 != 0 || g.Kg % 4 != 0 || g.K % 4 != 0 || g.Cg == 0 || g.Kg == 0) return false;
+  if (((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(dx)) & 15u) != 0) return false;
+  const long long out = static_cast<long long>(g.N) * g.Ho * g.Wo * g.K;
+  if (out == 0 || g.sh <= 0 || g.sw <= 0 || static_cast<long long>(g.sh) * g.sw > 65535) return false;
+  TileDxArgs a;
+  a.dy = dy; a.w = w; a.dx = dx; a.g = g;
+  a.rows = (g.H + g.sh - 1) / g.sh;
+  a.cgs = ((g.W + g.sw - 1) / g.sw + kTilePix - 1) / kTilePix;
+  a.groups = static_cast<long long>(g.N) * a.rows * a.cgs;
+  const int q = g.Cg / 4;
+  const int qb = q % 8 == 0 ? 8 : (q % 4 == 0 ? 4 : (q % 2 == 0 ? 2 : 1));
+  const long long z = g.C / (4 * qb);
+  if (a.groups >= (1LL << 31) - kDirectThreads || z > 65535) return false;
+  a.fd_rows = fastdiv_m(a.rows);
+  a.fd_cgs = fastdiv_m(a.cgs);
+  a.fd_sw = fastdiv_m(g.sw);
+  const int per = kDirectThreads / qb;
+  const dim3 grid(static_cast<unsigned>((a.groups + per - 1) / per), g.sh * g.sw, static_cast<unsigned>(z));
+  const dim3 block(kDirectThreads);
+  if (qb == 8) hipLaunchKernelGGL(f32_bprop_tile_kernel<8>, grid, block, 0, stream, a);
+  else if (qb == 4) hipLaunchKernelGGL(f32_bprop_tile_kernel<4>, grid, block, 0, stream, a);
+  else if (qb == 2) hipLaunchKernelGGL(f32_bprop_tile_kernel<2>, grid, block, 0, stream, a);
+  else hipLaunchKernelGGL(f32_bprop_tile_kernel<1>, grid, block, 0, stream, a);
+  return true;
+}
+
+}  // namespace
+
 hipError_t launch_f32_bprop_direct(const Geom& g, const BlockGeom& bg, const float* dy, const float* w, float* dx,
                                    hipStream_t stream) {
+  if (launch_bprop_tile(g, bg, dy, w, dx, stream)) return hipGetLastError();
   if (f32_bprop_direct4_eligible(g, w, dx)) {
     const long long quads = static_cast<long long>(g.N) * g.H * g.W * (g.C / 4);
     if (quads == 0) return hipSuccess;

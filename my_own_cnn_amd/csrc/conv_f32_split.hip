@@ -28,7 +28,9 @@
 //
 // Measured (us; before: the fp32 implicit GEMM of conv_f32.hip): 32 x 56 x 56, 64 -> 64 3x3 54-58
 // (110), its dx 58 (122); 32 x 28 x 28, 128 -> 256 97 (207), dx 97 (226), 2 x 4 filter blocks 93
-// (199); 16 x 64 x 64 dilated 32 (57); four groups of 32 64 (111); one 56 x 56 image 14.6 (30.6).
+// (199); 16 x 64 x 64 dilated 32 (57); four groups of 32 64 (111); one 56 x 56 image 13.1 (30.8).
+// Few tiles are bound by the stages' latency: 8 waves on 16 positions each (NSEG 1) halve the
+// stages of 4 waves on 32 (one image 15.4 -> 13.1, 4 x 16 x 16, 256 -> 64 42 -> 38).
 // Bound by the matrix instructions and the power they draw: with everything but the MFMAs and
 // their LDS reads taken out the 28 x 28 dx still took 67 us; the filter's split and stores cost 8,
 // its loads 8 and the halo 4.  The 56 x 56 layer loses a further 9 us per workgroup at its start
@@ -37,6 +39,7 @@
 #include "f32_split.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace miq {
@@ -587,8 +590,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     store_a();
     __syncthreads();
     if constexpr (MULTI) run_blocks();
-    else if (whole) run(std::integral_constant<int, NSEG>{});
-    else run(std::integral_constant<int, NSEG - 1>{});
+    else if (NSEG == 1 || whole) run(std::integral_constant<int, NSEG>{});
+    else run(std::integral_constant<int, NSEG == 1 ? 1 : NSEG - 1>{});
   }
 
   bool bad = mn < kSmall2;
@@ -607,7 +610,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   __syncthreads();
   if (*flag != 0) {
     // the tile again with fp32 MFMAs: per tap, 16 channels a step, gathered into LDS
-    constexpr int UR = BM * 4 / NT;
+    constexpr int UR = BM * 4 < NT ? 1 : BM * 4 / NT;
     v4f* const fA = reinterpret_cast<v4f*>(lds);
     v4f* const fB = fA + BM * 4;
     int uh[UR], uw[UR];
@@ -641,7 +644,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
           const int hi = uh[k] + r * g.dh, wi = uw[k] + s * g.dw;
           const bool ok = ch < g.Cg && hi >= ylo && hi < yhi && wi >= xlo && wi < xhi;
           const v4f v = *reinterpret_cast<const v4f*>(ok ? ux[k] + (static_cast<size_t>(hi) * g.W + wi) * g.C + ch : a.x);
-          fA[f32s_slot((t + NT * k) >> 2, t & 3)] = ok ? v : zero;
+          if (t + NT * k < BM * 4) fA[f32s_slot((t + NT * k) >> 2, t & 3)] = ok ? v : zero;
         }
         for (int u = t; u < BN * 4; u += NT) {
           const int kr = min(n0 + (u >> 2), g.Kg - 1);
@@ -723,7 +726,7 @@ struct SplitPlan {
 struct SplitVariant {
   int nseg, wm, wn;
 };
-constexpr SplitVariant kVariants[] = {{4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {4, 4, 1}};
+constexpr SplitVariant kVariants[] = {{4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {4, 4, 1}, {1, 4, 2}};
 
 // Estimated cycles of a launch: rounds of workgroups over the 256 CUs x (K-blocks at the MFMA rate
 // of a wave's tile, the staged values, a fixed start and end).
@@ -765,23 +768,28 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
     p.lds = static_cast<size_t>(3 * (co * p.hps + 8) + 2 * bsz) * 16 + static_cast<size_t>(p.nst * so + 1) * 4 +
             (blocked_dx ? 80 + 32 * kSplitMaxReach : 0);
     if (p.lds > kSplitLds) continue;
-    const int per_cu = std::max(1, std::min<int>({static_cast<int>(kSplitLds / p.lds), 8 / (V.wm * V.wn), 4}));
-    const double kb = static_cast<double>(p.nchunk) * ((p.noct + 3) / 4);
-    const double mfma = kb * V.nseg * 12 * 16.0 * V.wm * V.wn / 4;  // SIMD cycles of a workgroup
+    // workgroups that share a CU; a stage takes at least its filter values' way through the
+    // registers (1200 cycles with 4 waves, 1950 with 8, measured on one image), less when shared
+    const int fit = std::max(1, std::min<int>({static_cast<int>(kSplitLds / p.lds), 8 / (V.wm * V.wn), 4}));
+    const int per_cu = std::max(1, static_cast<int>(std::min<long long>(fit, (p.blocks + 255) / 256)));
+    const double least = (V.wm * V.wn >= 8 ? 1950.0 : 1200.0) / std::sqrt(static_cast<double>(per_cu));
+    const double kbs = V.nseg * 12 * 16.0 * V.wm * V.wn / 4 * 1.25;  // SIMD cycles of a K-block
+    const double mfma = p.nchunk * ((p.noct + 3) / 4) * kbs;
     const double stage = p.nchunk * (static_cast<double>(p.hp) * co + static_cast<double>(p.nst) * so * bn) * 60.0 / 64;
-    double wg = mfma * 1.25 + stage * 0.7 + 2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
+    double wg = p.nchunk * p.nst * std::max((p.noct + 3) / 4 * kbs / p.nst, least) + stage * 0.7 +
+                2500.0 * p.nchunk / per_cu + (2500.0 + 1000.0 * V.nseg) / per_cu;
     if (blocked_dx) {
       // a tile edge on a block edge adds the taps that cross it: (block, tap) pairs and blocks of
       // an average tile; a stage takes at least its filter values' way through the registers
       const double pairs = (g.R + (g.R - 1.0) / p.nty) * (g.S + (g.S - 1.0) / p.ntx);
       const double blks = (1 + (g.R > 1 ? 2.0 : 0.0) / p.nty) * (1 + (g.S > 1 ? 2.0 : 0.0) / p.ntx);
       const double stages = p.nchunk * (pairs * co / so + 0.5 * blks);
-      wg = std::max(mfma * 1.25, stages * 2200.0) + 0.3 * std::min(mfma, stages * 2200.0) + stage * 0.7 +
+      const double bleast = 1.13 * least;
+      wg = std::max(mfma, stages * bleast) + 0.24 * std::min(mfma, stages * bleast) + stage * 0.7 +
            2500.0 * p.nchunk / per_cu + 4000.0 / per_cu;
     }
     const double rounds = std::ceil(static_cast<double>(p.blocks) / (256.0 * per_cu)) * per_cu;
     p.cost = std::min(rounds, static_cast<double>(p.blocks) / 256.0 + 0.5 * per_cu) * wg;
-    if (p.blocks < 256) p.cost = wg;
     if (best->variant < 0 || p.cost < best->cost) *best = p;
   }
 }
@@ -791,13 +799,14 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
 // halo and a short reduction leaves the split unpaid (1x1 128 -> 256: 100 against 89 us; 512 -> 128
 // at 14 x 14: 24.5 against 28; transposed 256 -> 64: 43 against 59), and at most 32 output channels
 // at a stride give too few MFMAs per halo value (112 x 112, 32 -> 32: 39 against 35 us, 32 -> 64:
-// 24 against 31).
+// 24 against 31); four channels fill half an octet (8 x 30 x 30, 4 -> 32: 9.2 against 8.3 us).
 SplitPlan make_plan(const Geom& g, int rh, int rw, long long nreg, bool transposed) {
   SplitPlan best{};
   best.variant = -1;
   if (g.dh <= 0 || g.dw <= 0 || g.sh <= 0 || g.sw <= 0) return best;
   if (g.R * g.S == 1 && g.Cg < (transposed ? 128 : 256)) return best;
   if (g.Kg <= 32 && (g.sh > 1 || g.sw > 1)) return best;
+  if (g.Cg < 8 && g.R * g.S <= 9) return best;
   // 32-bit byte offsets: into a group's filter (every block of it) and into an image
   if (static_cast<double>(std::max(g.Kg, g.Cg)) * nreg * g.R * g.S * std::max(g.Kg, g.Cg) * 4 >= 2147483647.0 ||
       static_cast<double>(g.H) * g.W * g.C * 4 >= 2147483647.0) {
@@ -842,7 +851,10 @@ hipError_t launch_split(const SplitArgs& a, const SplitPlan& p, hipStream_t stre
     case 0: return launch_variant<MODE, 4, 4, 2>(a, p, stream);
     case 1: return launch_variant<MODE, 4, 2, 2>(a, p, stream);
     case 2: return launch_variant<MODE, 2, 2, 2>(a, p, stream);
-    default: return launch_variant<MODE, 4, 4, 1>(a, p, stream);
+    case 3: return launch_variant<MODE, 4, 4, 1>(a, p, stream);
+    default:
+      if constexpr (MODE != kSplitTransBlocked) return launch_variant<MODE, 1, 4, 2>(a, p, stream);
+      return hipErrorInvalidValue;
   }
 }
 
@@ -860,7 +872,7 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
   if (g.R * g.S == 1 && g.Cg < 128) return best;
   if (static_cast<double>(g.Kg) * nreg * g.R * g.S * g.Cg * 4 >= 2147483647.0) return best;
   for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
-    if ((kVariants[v].wn == 1) != (g.Kg <= 32)) continue;
+    if ((kVariants[v].wn == 1) != (g.Kg <= 32) || kVariants[v].nseg == 1) continue;
     const int bm = 16 * kVariants[v].nseg * kVariants[v].wm;
     for (const int images : {16, 8, 4, 2, 1}) {
       if (images > g.N && images != 1) continue;

@@ -28,6 +28,9 @@ CASES = [
     (1, 1, 3, 256, 300, 1, 1, (0, 0, 1, 1, 1, 1, 1)),    # one tap
     (1, 9, 130, 264, 32, 1, 1, (0, 0, 1, 1, 1, 1, 1)),
     (1, 6, 6, 16, 32, 3, 3, (3, 3, 1, 1, 1, 1, 1)),      # padding past the filter's reach
+    (24, 28, 28, 64, 96, 3, 3, (1, 1, 1, 1, 1, 1, 1)),   # enough tiles for the larger ones
+    (32, 14, 14, 64, 256, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (40, 30, 26, 32, 32, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
 ]
 
 

@@ -728,6 +728,11 @@ struct SplitVariant {
 };
 constexpr SplitVariant kVariants[] = {{4, 4, 2}, {4, 2, 2}, {2, 2, 2}, {4, 4, 1}, {1, 4, 2}};
 
+// a reduction and an image to run over; an empty one is all zeros, which the implicit GEMM writes
+bool plain_extents(const Geom& g) {
+  return g.N > 0 && g.H > 0 && g.W > 0 && g.Cg > 0 && g.Kg > 0 && g.R > 0 && g.S > 0;
+}
+
 // Estimated cycles of a launch: rounds of workgroups over the 256 CUs x (K-blocks at the MFMA rate
 // of a wave's tile, the staged values, a fixed start and end).
 void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int th, int tw, int twp,
@@ -803,7 +808,7 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
 SplitPlan make_plan(const Geom& g, int rh, int rw, long long nreg, bool transposed) {
   SplitPlan best{};
   best.variant = -1;
-  if (g.dh <= 0 || g.dw <= 0 || g.sh <= 0 || g.sw <= 0) return best;
+  if (!plain_extents(g) || g.dh <= 0 || g.dw <= 0 || g.sh <= 0 || g.sw <= 0) return best;
   if (g.R * g.S == 1 && g.Cg < (transposed ? 128 : 256)) return best;
   if (g.Kg <= 32 && (g.sh > 1 || g.sw > 1)) return best;
   if (g.Cg < 8 && g.R * g.S <= 9) return best;
@@ -868,7 +873,7 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
   SplitPlan best{};
   best.variant = -1;
   const long long nreg = static_cast<long long>(bg.By) * bg.Bx;
-  if (g.dh <= 0 || g.dw <= 0 || g.R > 16 || g.S > 16) return best;
+  if (!plain_extents(g) || g.dh <= 0 || g.dw <= 0 || g.R > 16 || g.S > 16) return best;
   if (g.R * g.S == 1 && g.Cg < 128) return best;
   if (static_cast<double>(g.Kg) * nreg * g.R * g.S * g.Cg * 4 >= 2147483647.0) return best;
   for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {

@@ -69,6 +69,16 @@ def test_forward_and_dx(device, case):
     check(dx.cpu(), want, mag, r * s * k // conv[6])
 
 
+@pytest.mark.parametrize("taps", [3, 5])
+def test_empty_reductions_are_zero(device, taps):
+    y = M.conv2d_nhwc_f32(torch.empty((1, 8, 8, 0), device=device), torch.empty((40, taps, taps, 0), device=device))
+    assert float(y.abs().max()) == 0.0
+    dx = torch.full((1, 8, 8, 16), 7.0, device=device)
+    M.launch_bprop_nhwc(torch.empty((1, 8, 8, 0), device=device), torch.empty((0, taps, taps, 16), device=device), dx,
+                        1, 8, 8, 16, taps, taps, 0, (taps // 2, taps // 2, 1, 1, 1, 1, 1))
+    assert float(dx.abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("grid", [(2, 3), (4, 2)])
 def test_blocked_forward(device, grid):
     n, h, w, c, k = 3, 16, 18, 40, 70

@@ -571,31 +571,46 @@ __global__ void __launch_bounds__(kDirectThreads) f32_depthwise_kernel(const flo
   store_gap(acc);
 }
 
-// Depthwise fp32 dw (C/groups == K/groups == 1, C % 4 == 0, R*S <= 16): one thread per 4
-// channels and a run of kDwGradPix consecutive output pixels, summing x * dy for all R*S taps
-// in registers (float4 reads of x and dy).  With `part` the thread stores its partial sums at
-// part[run][c][tap] (every entry of every run is written) and f32_sum_parts_kernel adds the
-// runs in order: the same result on every call.  Without it they are added into dw (zeroed
-// first) with float atomics, whose order varies from run to run.  Either order differs from
-// cpu_grad_nhwc's.
+// Depthwise fp32 dw (C/groups == K/groups == 1, C % 4 == 0, R*S <= 16).  A workgroup takes
+// kDwGradPix consecutive output pixels and 128 channels: thread (sub, quad) sums x * dy for all R*S
+// taps of 4 channels over 16 of the pixels in registers (float4 reads of x and dy), and the 8 subs'
+// sums are added in order through LDS.  With `part` they are stored at part[run][c][tap] (every
+// entry of every run is written) and f32_sum_parts_kernel adds the runs in order: the same result
+// on every call.  Without it they are added into dw (zeroed first) with float atomics, whose order
+// varies from run to run.  Either order differs from cpu_grad_nhwc's.
+// Bound by load latency: one thread per 128 pixels gave 392 waves on 32 x 56 x 56 x 128, less than
+// one per SIMD, each tap's load behind its bounds branch; now 3136 waves, and every load of a pixel
+// is issued before its sums.  With the sum of the runs, 32 x 56 x 56 x 128 3x3: 346 -> 76 us (x and
+// dy once: 21 us), 17 x 75 x 72 x 64: 327 -> 47, 8 x 25 x 25 x 32: 242 -> 28, 4 x 4 taps on
+// 2 x 30 x 30 x 36: 406 -> 52.  Up to 9 taps have their own instance (36 registers of sums, not 64).
 constexpr int kDwGradPix = 128;
 constexpr int kDwGradTaps = 16;
+constexpr int kDwGradQuads = 32;                            // channel quads per workgroup
+constexpr int kDwGradSubs = kDirectThreads / kDwGradQuads;  // pixel runs per workgroup
 
+template <int TAPS>
 __global__ void __launch_bounds__(kDirectThreads) f32_depthwise_grad_kernel(const float* __restrict__ x,
                                                                             const float* __restrict__ dy,
                                                                             float* __restrict__ dw,
-                                                                            float* __restrict__ part, Geom g, int P,
-                                                                            long long total) {
-  const long long e = static_cast<long long>(blockIdx.x) * kDirectThreads + threadIdx.x;
-  if (e >= total) return;
-  const int c4n = g.C / 4;
-  const int c = 4 * static_cast<int>(e % c4n);
-  const int p0 = static_cast<int>(e / c4n) * kDwGradPix;
-  const int p1 = min(P, p0 + kDwGradPix);
+                                                                            float* __restrict__ part, Geom g, int P) {
+  __shared__ v4f sums[kDirectThreads];
+  const int quad = blockIdx.y * kDwGradQuads + threadIdx.x % kDwGradQuads;
+  const int sub = threadIdx.x / kDwGradQuads;
+  const bool live = quad < g.C / 4;
+  const int c = live ? 4 * quad : 0;
+  const int run0 = blockIdx.x * kDwGradPix;
+  const int p0 = run0 + sub * (kDwGradPix / kDwGradSubs);
+  const int p1 = min(P, p0 + kDwGradPix / kDwGradSubs);
   const int taps = g.R * g.S;
-  v4f acc[kDwGradTaps];
+  v4f acc[TAPS];
+  int tr[TAPS], ts[TAPS];
 #pragma unroll
-  for (int t = 0; t < kDwGradTaps; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < TAPS; ++t) {
+    acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    const int r = t / g.S;
+    tr[t] = r * g.dh - g.ph;
+    ts[t] = (t - r * g.S) * g.dw - g.pw;
+  }
   const int hw = g.Ho * g.Wo;
   int n = p0 / hw;
   int ho = (p0 - n * hw) / g.Wo;
@@ -603,20 +618,21 @@ __global__ void __launch_bounds__(kDirectThreads) f32_depthwise_grad_kernel(cons
   for (int p = p0; p < p1; ++p) {
     const v4f dv = *reinterpret_cast<const v4f*>(dy + static_cast<size_t>(p) * g.K + c);
     const float* xn = x + static_cast<size_t>(n) * g.H * g.W * g.C + c;
+    v4f xv[TAPS];
+    bool ok[TAPS];
 #pragma unroll
-    for (int t = 0; t < kDwGradTaps; ++t) {
-      if (t < taps) {
-        const int r = t / g.S;
-        const int s = t - r * g.S;
-        const int hi = ho * g.sh - g.ph + r * g.dh;
-        const int wi = wo * g.sw - g.pw + s * g.dw;
-        if (hi >= 0 && hi < g.H && wi >= 0 && wi < g.W) {
-          const v4f xv = *reinterpret_cast<const v4f*>(xn + (static_cast<size_t>(hi) * g.W + wi) * g.C);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[t][j] = __fadd_rn(acc[t][j], __fmul_rn(xv[j], dv[j]));
-        }
-      }
+    for (int t = 0; t < TAPS; ++t) {
+      const int hi = ho * g.sh + tr[t], wi = wo * g.sw + ts[t];
+      ok[t] = t < taps && hi >= 0 && hi < g.H && wi >= 0 && wi < g.W;
+      xv[t] = *reinterpret_cast<const v4f*>(xn + (ok[t] ? (static_cast<size_t>(hi) * g.W + wi) * g.C : 0));
     }
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float v = __fadd_rn(acc[t][j], __fmul_rn(xv[t][j], dv[j]));
+        acc[t][j] = ok[t] ? v : acc[t][j];  // a tap outside the image adds nothing
+      }
     if (++wo == g.Wo) {
       wo = 0;
       if (++ho == g.Ho) {
@@ -625,20 +641,27 @@ __global__ void __launch_bounds__(kDirectThreads) f32_depthwise_grad_kernel(cons
       }
     }
   }
-  if (part != nullptr) {
-    float* pr = part + static_cast<size_t>(p0 / kDwGradPix) * g.C * taps;
 #pragma unroll
-    for (int t = 0; t < kDwGradTaps; ++t)
-      if (t < taps)
+  for (int t = 0; t < TAPS; ++t) {
+    if (t < taps) {  // uniform
+      sums[threadIdx.x] = acc[t];
+      __syncthreads();
+      if (sub == 0 && live) {
+        v4f v = acc[t];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) pr[static_cast<size_t>(c + j) * taps + t] = acc[t][j];
-    return;
+        for (int u = 1; u < kDwGradSubs; ++u)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = __fadd_rn(v[j], sums[u * kDwGradQuads + threadIdx.x][j]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const size_t at = static_cast<size_t>(c + j) * taps + t;
+          if (part != nullptr) part[static_cast<size_t>(blockIdx.x) * g.C * taps + at] = v[j];
+          else unsafeAtomicAdd(dw + at, v[j]);
+        }
+      }
+      __syncthreads();  // sums is free for the next tap
+    }
   }
-#pragma unroll
-  for (int t = 0; t < kDwGradTaps; ++t)
-    if (t < taps)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) unsafeAtomicAdd(dw + static_cast<size_t>(c + j) * taps + t, acc[t][j]);
 }
 
 // dw[i] = the sum of part[0][i] .. part[nparts - 1][i] (`count` elements per part) in a fixed
@@ -1653,6 +1676,7 @@ hipError_t launch_f32_direct(const Geom& g, const BlockGeom& bg, const float* x,
 bool f32_depthwise_grad_eligible(const Geom& g, const void* x, const void* dy) {
   return g.Cg == 1 && g.Kg == 1 && g.C % 4 == 0 && g.R * g.S <= kDwGradTaps && g.R * g.S > 0 && g.H > 0 &&
          g.W > 0 && static_cast<long long>(g.N) * g.Ho * g.Wo < (1LL << 31) - kDwGradPix &&
+         g.C <= 4 * kDwGradQuads * 65535 &&  // the grid's y
          (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(dy) & 15u) == 0;
 }
 
@@ -1668,17 +1692,17 @@ hipError_t launch_f32_depthwise_grad(const Geom& g, const float* x, const float*
   const int P = g.N * g.Ho * g.Wo;
   const long long count = static_cast<long long>(g.K) * g.R * g.S;
   const long long runs = (static_cast<long long>(P) + kDwGradPix - 1) / kDwGradPix;
-  const long long total = runs * (g.C / 4);
   if (!ordered || runs == 0) {
     const unsigned zb = static_cast<unsigned>(std::min<long long>((count + kDirectThreads - 1) / kDirectThreads, 4096));
     hipLaunchKernelGGL(f32_zero_kernel, dim3(zb), dim3(kDirectThreads), 0, stream, dw, count);
   }
-  if (total == 0) return hipGetLastError();
-  const long long blocks = (total + kDirectThreads - 1) / kDirectThreads;
+  if (runs * g.C == 0) return hipGetLastError();
   // ordered: one run writes dw directly; more write their partial sums, added in run order
   float* part = !ordered ? nullptr : (runs == 1 ? dw : ws);
-  hipLaunchKernelGGL(f32_depthwise_grad_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kDirectThreads), 0, stream,
-                     x, dy, dw, part, g, P, total);
+  const dim3 grid(static_cast<unsigned>(runs), static_cast<unsigned>((g.C / 4 + kDwGradQuads - 1) / kDwGradQuads));
+  const dim3 block(kDirectThreads);
+  if (g.R * g.S <= 9) hipLaunchKernelGGL(f32_depthwise_grad_kernel<9>, grid, block, 0, stream, x, dy, dw, part, g, P);
+  else hipLaunchKernelGGL(f32_depthwise_grad_kernel<kDwGradTaps>, grid, block, 0, stream, x, dy, dw, part, g, P);
   if (ordered && runs > 1) launch_sum_parts(ws, dw, count, runs, stream);
   return hipGetLastError();
 }

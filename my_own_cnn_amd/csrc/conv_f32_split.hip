@@ -1,19 +1,18 @@
 // fp32 NHWC convolution on the bf16 matrix cores, without losing fp32 accuracy: the forward pass
 // and, read with the flipped, channel-transposed filter, the dx of a stride-1 convolution.
 //
-// Arithmetic.  Each operand is split into three bf16 numbers, x = x0 + x1 + x2 (round to nearest
-// even at each step: 8 + 8 + 8 significant bits hold all 24 of an fp32 value of magnitude 2^-110
-// and more).  A product is the six terms x2 w0, x0 w2, x1 w1, x0 w1, x1 w0, x0 w0; the dropped
+// Arithmetic.  Each operand is scaled by 2^23 and split into three bf16 numbers, x = x0 + x1 + x2
+// (round to nearest even at each step: 8 + 8 + 8 significant bits hold all 24 of an fp32 value, and
+// the scale keeps the pieces of the smallest ones normal).  A product is the six terms x2 w0, x0 w2, x1 w1, x0 w1, x1 w0, x0 w0; the dropped
 // ones are below 2^-26 of it.  The terms of 32 reduction values sum from zero in that order, and
 // the sum is added to the fp32 accumulator.  Error against 64 bits, K = 576 / 4608 normal
 // inputs: 0.9e-7 / 2.3e-7 relative, where a chain of v_mfma_f32_16x16x4f32 gives 4.4e-7 / 1.2e-6
 // (one rounding of the running sum per 32 products, not per 4).  Six
 // v_mfma_f32_16x16x32_bf16 issue in 0.38 of the time of the eight v_mfma_f32_16x16x4f32 they
 // replace; a loop of them alone sustains 1680 TFLOP/s on this card, 280 of them the convolution's.
-// Inputs the split does not carry are found at run time and their whole tile is computed again
-// with v_mfma_f32_16x16x4f32: a nonzero value below 2^-110 (checked as the values are staged), and
-// anything that makes a stored result infinite or NaN (an infinite or NaN input, or a value that
-// rounds up to a bf16 infinity).
+// What the split does not carry is found at the end of a tile, as a result that is infinite or NaN,
+// and the whole tile is computed again with v_mfma_f32_16x16x4f32: an infinite or NaN input, an
+// input of 2^105 or more, a scaled sum past the fp32 range (a result of 2^82 or more).
 //
 // Work.  A workgroup computes a tile of ti images x th x tw output positions (at most
 // 16 NSEG WM) and 32 WN channels of one group; wave (wm, wn) computes 16 NSEG of the positions
@@ -241,7 +240,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
 
   v4f va[kSplitUnits][2];
   v4f vb[MULTI ? 2 : 1][BU][2];  // filter values in flight, MULTI: of two stages
-  unsigned mn = 0xffffffffu;
   const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
   auto load_a = [&](int c) {
     const int c0 = 8 * a.co * c;
@@ -256,7 +254,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
 #pragma unroll
     for (int j = 0; j < kSplitUnits; ++j) {
       if (aput[j] != ~0u) {
-        const Split8 s = split8(va[j][0], va[j][1], mn);
+        const Split8 s = split8(va[j][0], va[j][1], kSplitScale);
         v4u* const d = sA + (aput[j] & 0xfffffu);
 #pragma unroll
         for (int p = 0; p < 3; ++p) d[p] = s.p[p];
@@ -363,7 +361,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     constexpr int V = MULTI ? decltype(set)::value : 0;
 #pragma unroll
     for (int j = 0; j < BU; ++j) {
-      const Split8 sp = split8(vb[V][j][0], vb[V][j][1], mn);
+      const Split8 sp = split8(vb[V][j][0], vb[V][j][1], kSplitScale);
 #pragma unroll
       for (int p = 0; p < 3; ++p) sB[buf * BSZ + bslot[j] + p] = sp.p[p];
     }
@@ -594,7 +592,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     else run(std::integral_constant<int, NSEG == 1 ? 1 : NSEG - 1>{});
   }
 
-  bool bad = mn < kSmall2;
+  bool bad = false;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -603,7 +601,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       const bool ok = i < own && decode(m0 + 16 * i, im, lr, lc);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        bad |= ok && !(__builtin_fabsf(acc[j][i][e]) <= 3.4028234663852886e38f);
+        bad |= ok && !(__builtin_fabsf(acc[j][i][e]) <= kFltMax);
       }
     }
   if (bad) *flag = 1;
@@ -678,6 +676,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
               acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][k], fa[i][k], acc[j][i], 0, 0, 0);
       }
     }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < NSEG; ++i) acc[j][i] *= kSplitUnscale;
   }
 
   // lane (c = lane % 16, q): position c of each segment, channels 4 q .. 4 q + 3 of each 16

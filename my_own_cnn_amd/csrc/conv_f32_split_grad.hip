@@ -149,7 +149,6 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
   const int xput = (t / OX) * a.recx + 16 * (t % OX), yput = (t / OY) * a.recy + 16 * (t % OY);
 
   v4f vx[UX][2], vy[UY][2];
-  unsigned mn = 0xffffffffu;
   const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
   auto tile_at = [&](int ti_, int& img0, int& ty0, int& tx0) {
     const int q1 = fdiv(ti_, a.fd_ntx);
@@ -192,14 +191,14 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
 #pragma unroll
     for (int j = 0; j < UX; ++j)
       if (xat[j] != kOut) {
-        const Split8 s = split8(vx[j][0], vx[j][1], mn);
+        const Split8 s = split8(vx[j][0], vx[j][1], kSplitScale);
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<v4u*>(bx + j * PX * a.recx + 2 * CH * p) = s.p[p];
       }
 #pragma unroll
     for (int j = 0; j < UY; ++j)
       if (t / OY + PY * j < 32 * a.kbs) {
-        const Split8 s = split8(vy[j][0], vy[j][1], mn);
+        const Split8 s = split8(vy[j][0], vy[j][1], kSplitScale);
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<v4u*>(by + j * PY * a.recy + 2 * KR * p) = s.p[p];
       }
@@ -303,7 +302,7 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
   }
   reduce();
 
-  bool bad = mn < kSmall2;
+  bool bad = false;
   if (wp == 0) {
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -311,7 +310,7 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) bad |= !(__builtin_fabsf(acc[b][i][e]) <= 3.4028234663852886e38f);
+          for (int e = 0; e < 4; ++e) bad |= !(__builtin_fabsf(acc[b][i][e]) <= kFltMax);
       }
   }
   if (bad) *flag = 1;
@@ -354,6 +353,12 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
     }
     __syncthreads();
     reduce();
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      acc[b][0] *= kSplitUnscale;
+      acc[b][1] *= kSplitUnscale;
+    }
   }
 
   // lane (n16, q) of a tile: output channels 4 q .. 4 q + 3, input channel n16

@@ -12,23 +12,24 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitLds = 160 * 1024;           // bytes per CU
-constexpr unsigned kSmall2 = (17u << 24) - 1u;  // 2 * bits(2^-110) - 1
+constexpr float kSplitScale = 8388608.0f;       // 2^23: the scale of staged values
+constexpr float kSplitUnscale = 0x1p-46f;       // of a product's two
+constexpr float kFltMax = 3.4028234663852886e38f;
 constexpr unsigned kNone = 0x80000000u;         // a buffer offset that reads zero
 
 struct Split8 {
   v4u p[3];
 };
 
-// Eight fp32 values as three bf16 each; `mn` collects the smallest 2 * bits - 1 (zero wraps to the
-// largest unsigned value).
-__device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, unsigned& mn) {
+// Eight fp32 values times `scale` as three bf16 each.  With a scale of 2^23 every fp32 value below
+// 2^105 is carried exactly, subnormals among them: a residual of the scaled value is a multiple of
+// 2^-126, so each piece is zero or a normal bf16, and the corrections of a product that fp32 holds
+// stay above the subnormal range.  A larger value becomes infinite, and whatever it reaches infinite or NaN.
+__device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, float scale) {
   Split8 out;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const v2f v = j < 2 ? v2f{lo[2 * j], lo[2 * j + 1]} : v2f{hi[2 * j - 4], hi[2 * j - 3]};
-    const unsigned u0 = (__builtin_bit_cast(unsigned, static_cast<float>(v[0])) << 1) - 1u;
-    const unsigned u1 = (__builtin_bit_cast(unsigned, static_cast<float>(v[1])) << 1) - 1u;
-    mn = min(mn, min(u0, u1));
+    const v2f v = j < 2 ? v2f{lo[2 * j] * scale, lo[2 * j + 1] * scale} : v2f{hi[2 * j - 4] * scale, hi[2 * j - 3] * scale};
     const v2b h = __builtin_convertvector(v, v2b);
     const v2f r1 = v2f{v[0] - static_cast<float>(h[0]), v[1] - static_cast<float>(h[1])};
     const v2b m = __builtin_convertvector(r1, v2b);

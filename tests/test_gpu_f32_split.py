@@ -135,8 +135,8 @@ def test_blocked_dx(device, case):
     dy = torch.randn((n, ho, wo, k), generator=gen)
     dx = torch.full((n, h, w, c), 7.0, device=device)
     for special in (False, True):
-        if special:  # one value sends its tiles through the fp32 instructions
-            dy[0, ho // 2, wo // 2, 1] = 2.0 ** -130
+        if special:  # one value past the scaled range sends its tiles through the fp32 instructions
+            dy[0, ho // 2, wo // 2, 1] = 2.0 ** 112
         M.launch_block_bprop_nhwc(dy.to(device), wt.to(device), dx, n, h, w, c, r, s, k, p)
         want, mag = blocked_dx(dy, wt, (n, h, w, c), conv)
         check(dx.cpu(), want, mag, r * s * k // conv[6])
@@ -176,6 +176,69 @@ def test_small_inputs(device, scale):
     want, = torch.autograd.grad(conv64(xg, wt, case[7]), xg, dy.double())
     mag, = torch.autograd.grad(conv64(xg, wt.abs(), case[7]), xg, dy.double().abs())
     check(dx.cpu(), want, mag, 9 * 36)
+
+
+@pytest.mark.parametrize("tiny", [1e-35, 1e-40, 2.0 ** -149])
+def test_a_tiny_value_leaves_the_other_results(device, tiny):
+    """Every fp32 value is carried by the split: a tile that holds a tiny one keeps the bits of the
+    results that the value does not reach."""
+    n, h, w, c, k = 2, 20, 20, 40, 72
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    bp = M.BlockConv2DParams(M.Conv2DParams(*conv), 2, 2)
+    gen = torch.Generator().manual_seed(14)
+    x, wt = torch.randn((n, h, w, c), generator=gen), torch.randn((k, 3, 3, c), generator=gen)
+    dy, wb = torch.randn((n, h, w, k), generator=gen), torch.randn((k, 2, 2, 3, 3, c), generator=gen)
+
+    def outputs(x, wt, dy):
+        x, wt, dy = x.to(device), wt.to(device), dy.to(device)
+        y, dx, dxb, dw = torch.empty_like(dy), torch.empty_like(x), torch.empty_like(x), torch.empty_like(wt)
+        M.launch_fprop_nhwc(x, wt, y, n, h, w, c, 3, 3, k, conv)
+        M.launch_bprop_nhwc(dy, wt, dx, n, h, w, c, 3, 3, k, conv)
+        M.launch_block_bprop_nhwc(dy, wb.to(device), dxb, n, h, w, c, 3, 3, k, bp)
+        M.launch_grad_nhwc(x, dy, dw, n, h, w, c, 3, 3, k, conv)
+        return y.cpu(), dx.cpu(), dxb.cpu(), dw.cpu()
+
+    def put(t, at, v):
+        t = t.clone()
+        t[at] = v
+        return t
+
+    at, near = (1, 8, 9, 5), (1, slice(7, 10), slice(8, 11))
+    zero, got = (outputs(put(x, at, v), wt, dy) for v in (0.0, tiny))
+    for a, b, skip in ((zero[0], got[0], near), (zero[3], got[3], (slice(None), slice(None), slice(None), 5))):
+        assert torch.equal(put(a, skip, 0.0), put(b, skip, 0.0))
+    zero, got = (outputs(x, wt, put(dy, at, v)) for v in (0.0, tiny))
+    for i, skip in ((1, near), (2, near), (3, 5)):
+        assert torch.equal(put(zero[i], skip, 0.0), put(got[i], skip, 0.0)), i
+    zero, got = (outputs(x, put(wt, (7, 0, 2, 3), v), dy) for v in (0.0, tiny))
+    for i in (0, 1):
+        assert torch.equal(put(zero[i], (..., 7 if i == 0 else 3), 0.0), put(got[i], (..., 7 if i == 0 else 3), 0.0)), i
+
+
+@pytest.mark.parametrize("exp", [-55, -60, -63, -65, -70])
+def test_subnormal_products(device, exp):
+    """Both operands small: products and results reach the subnormal range, where each result (of
+    dw: each of its partial sums) is rounded to a multiple of 2^-149 once."""
+    n, h, w, c, k = 2, 24, 24, 32, 64
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    x, wt = data((n, h, w, c, k, 3, 3, conv), 16)
+    dy = torch.randn((n, h, w, k), generator=torch.Generator().manual_seed(17))
+    x, wt, dy = x * 2.0 ** exp, wt * 2.0 ** exp, dy * 2.0 ** exp
+    y, dx, dw = (torch.full(t.shape, 7.0, device=device) for t in (dy, x, wt))
+    dims = (n, h, w, c, 3, 3, k, conv)
+    M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims)
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims)
+    M.launch_grad_nhwc(x.to(device), dy.to(device), dw, *dims)
+    xg = x.double().requires_grad_()
+    want_dx, = torch.autograd.grad(conv64(xg, wt, conv), xg, dy.double())
+    mag_dx, = torch.autograd.grad(conv64(xg, wt.abs(), conv), xg, dy.double().abs())
+    parts = n * h * w // 64 + 1  # at most one partial sum per tile of positions
+    for got, want, mag, kdim, roundings in (
+            (y, conv64(x, wt, conv), conv64(x.abs(), wt.abs(), conv), 9 * c, 1),
+            (dx, want_dx, mag_dx, 9 * k, 1),
+            (dw, grad_want(x, dy, wt.shape, conv), grad_want(x, dy, wt.shape, conv, torch.abs), n * h * w + 512, parts)):
+        err = (got.cpu().double() - want).abs()
+        assert bool((err <= (kdim / 32 + 16) * 2.0 ** -23 * mag + roundings * 2.0 ** -150).all()), float(err.max())
 
 
 # filter gradients: (n, h, w, c, k, r, s, conv); channel counts on both sides of the wave layouts

@@ -10,6 +10,9 @@
 // (one rounding of the running sum per 32 products, not per 4).  Six
 // v_mfma_f32_16x16x32_bf16 issue in 0.38 of the time of the eight v_mfma_f32_16x16x4f32 they
 // replace; a loop of them alone sustains 1680 TFLOP/s on this card, 280 of them the convolution's.
+// The matrix core's sums lean towards minus infinity by a part of their last bit (a mean error of 0.3
+// of its rms at K = 576): half of the stages compute on negated filter values, and the running sums
+// change sign with them (a mean of at most 0.04).
 // What the split does not carry is found at the end of a tile, as a result that is infinite or NaN,
 // and the whole tile is computed again with v_mfma_f32_16x16x4f32: an infinite or NaN input, an
 // input of 2^105 or more, a scaled sum past the fp32 range (a result of 2^82 or more).
@@ -72,6 +75,7 @@ struct SplitArgs {
   int nchunk;
   int noct;        // R * S * co
   int nst;         // stages per chunk
+  int flip;        // stages between changes of sign
   int ow_taps, ow_cg;  // transposed filter: R * S and channels per group of the original
   int rx, nreg, rh, rw;  // output regions of rh x rw positions, rx per row (forward: the filter blocks)
   int By, Bx, bias_mode;
@@ -357,11 +361,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   };
-  auto store_b = [&](auto set, int buf) {  // the values of the set's last load_b
+  auto store_b = [&](auto set, int buf, float scale) {  // the values of the set's last load_b
     constexpr int V = MULTI ? decltype(set)::value : 0;
 #pragma unroll
     for (int j = 0; j < BU; ++j) {
-      const Split8 sp = split8(vb[V][j][0], vb[V][j][1], kSplitScale);
+      const Split8 sp = split8(vb[V][j][0], vb[V][j][1], scale);
 #pragma unroll
       for (int p = 0; p < 3; ++p) sB[buf * BSZ + bslot[j] + p] = sp.p[p];
     }
@@ -380,6 +384,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   // steps of up to two segments; a step's fragments are read while the step before it computes.
   // The six products of a step sum from zero, smallest first, and are added to the accumulators.
   int lc = 0, ls = 0;  // stage of the next load_b
+  float scale = kSplitScale;  // of the filter values stored last
+  int left = a.flip;          // stages until the sign turns
   Reach lb;
   set_reach(lb, 0);
   const int first_reach = lb.idx;
@@ -408,6 +414,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     for (int c = 0; c < a.nchunk; ++c) {
       const bool more = c + 1 < a.nchunk;
       for (int s = 0; s < a.nst; ++s) {
+        const bool turn = --left == 0;
+        if (turn) {
+          scale = -scale;
+          left = a.flip;
+        }
         int ao[SO / 4];
 #pragma unroll
         for (int kb = 0; kb < SO / 4; ++kb) ao[kb] = tab[SO * s + 4 * kb + q];
@@ -449,7 +460,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
               }
           }
           if constexpr (st == 0) {
-            store_b(even, buf ^ 1);
+            store_b(even, buf ^ 1, scale);
             fetch(even);
             if (s == 0) load_a(more ? c + 1 : c);
           }
@@ -468,6 +479,12 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
             step(std::integral_constant<int, HALVES>{});
             if constexpr (HALVES > 1) step(std::integral_constant<int, HALVES + 1>{});
           }
+        }
+        if (turn) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < NS; ++i) acc[j][i] = -acc[j][i];
         }
         __syncthreads();
         buf ^= 1;
@@ -507,7 +524,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     // stage s of the block: the filter buffer and register set of its parity over all stages
     auto stage = [&](auto par, auto other, int c, int s) {
       constexpr int PAR = decltype(par)::value;
-      store_b(other, PAR ^ 1);
+      store_b(other, PAR ^ 1, PAR ? kSplitScale : -kSplitScale);  // buffer 1 is negated
       fetch(other);
       if (s == 0 && rb.idx == first_reach) load_a(min(c + 1, a.nchunk - 1));
 #pragma unroll
@@ -551,7 +568,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
 #pragma unroll
               for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[j][i0 + i] += z[j][i];
+                for (int j = 0; j < 2; ++j) acc[j][i0 + i] = PAR ? acc[j][i0 + i] - z[j][i] : acc[j][i0 + i] + z[j][i];
             }
           }
         }
@@ -583,7 +600,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     fetch(even);
     load_a(0);
     if constexpr (MULTI) fetch(odd);
-    store_b(even, 0);
+    store_b(even, 0, scale);
     fetch(even);
     store_a();
     __syncthreads();
@@ -677,10 +694,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   } else {
+    const float unscale = scale < 0.0f ? -kSplitUnscale : kSplitUnscale;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int i = 0; i < NSEG; ++i) acc[j][i] *= kSplitUnscale;
+      for (int i = 0; i < NSEG; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[j][i][e] = __builtin_fmaf(acc[j][i][e], unscale, 0.0f);  // a zero sum is +0
   }
 
   // lane (c = lane % 16, q): position c of each segment, channels 4 q .. 4 q + 3 of each 16
@@ -922,6 +942,7 @@ bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const 
   a.ti = p.ti; a.th = p.th; a.tw = p.tw; a.hh = p.hh; a.hw = p.hw; a.hp = p.hp; a.hps = p.hps;
   a.twp = p.twp; a.ash = p.ash; a.lgh = p.co == 2 ? 0 : (p.co == 4 ? 1 : (p.co == 8 ? 2 : -1));
   a.co = p.co; a.nchunk = p.nchunk; a.noct = p.noct; a.nst = p.nst;
+  a.flip = split_flip(static_cast<long long>(p.nchunk) * p.nst);
   a.ow_taps = g.R * g.S;
   a.ow_cg = g.Kg;
   a.rx = bg.Bx; a.nreg = nreg; a.rh = rh; a.rw = rw;

@@ -273,6 +273,31 @@ def test_filter_gradient(device, case):
     check(dw.cpu(), grad_want(x, dy, wt.shape, conv), grad_want(x, dy, wt.shape, conv, torch.abs), dy[..., 0].numel() + 512)
 
 
+@pytest.mark.parametrize("shape", [(8, 40, 40, 64, 64), (8, 40, 40, 32, 32), (2, 40, 40, 96, 40)])
+def test_errors_do_not_lean(device, shape):
+    """The errors of a result's elements cancel: their mean is a small part of their rms.  The sums of
+    the matrix core alone lean one way (means of 0.3 rms forward, 0.8 in the filter gradient).  Over
+    N = 36,864 elements and more, independent errors give a mean of N^-1/2 = 0.005 rms; a step left over
+    from an odd count of them leans by a ninth of the 0.3."""
+    n, h, w, c, k = shape
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    gen = torch.Generator().manual_seed(18)
+    x, wt = torch.randn((n, h, w, c), generator=gen).clamp(min=0), torch.randn((k, 3, 3, c), generator=gen)
+    dy, wb = torch.randn((n, h, w, k), generator=gen), torch.randn((k, 2, 2, 3, 3, c), generator=gen)
+    dims = (n, h, w, c, 3, 3, k)
+    y, dx, dxb, dw = (torch.empty(t.shape, device=device) for t in (dy, x, x, wt))
+    M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims, conv)
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims, conv)
+    M.launch_block_bprop_nhwc(dy.to(device), wb.to(device), dxb, *dims, M.BlockConv2DParams(M.Conv2DParams(*conv), 2, 2))
+    M.launch_grad_nhwc(x.to(device), dy.to(device), dw, *dims, conv)
+    xg = x.double().requires_grad_()
+    want_dx, = torch.autograd.grad(conv64(xg, wt, conv), xg, dy.double())
+    for name, got, want in (("y", y, conv64(x, wt, conv)), ("dx", dx, want_dx), ("blocked dx", dxb, blocked_dx(dy, wb, x.shape, conv)[0]),
+                            ("dw", dw, grad_want(x, dy, wt.shape, conv))):
+        err = got.cpu().double() - want
+        assert abs(float(err.mean())) <= 0.1 * float(err.square().mean().sqrt()), name
+
+
 @pytest.mark.parametrize("grid", [(2, 3), (4, 1)])
 def test_blocked_filter_gradient(device, grid):
     n, h, w, c, k = 5, 16, 18, 40, 70

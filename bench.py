@@ -260,6 +260,7 @@ BLOCKED_SUITE = [
     ("blocked_small_batch_b4x4", 1, 56, 56, 64, 64, 3, 3, (1, 1, 1, 1, 1, 1, 1), 4, 4),
 ]
 PEAK_FP32_TFLOPS = 157.3  # dense fp32 MFMA, MI355X
+PEAK_SPLIT_TFLOPS = 2500.0 / 6  # dense bf16 MFMA, six products per fp32 one (split operands)
 
 
 def bench_fp32(args) -> None:
@@ -376,18 +377,22 @@ def bench_fp32(args) -> None:
         ms = t0.elapsed_time(t1) / args.steps
         flops = 2.0 * n * ho * wo * k * r * s_ * (c // g)  # conv_flops, src/main.cpp:143-145
         nbytes = 4.0 * (x.numel() + wt.numel() + y.numel())
-        t_mfma = flops / (PEAK_FP32_TFLOPS * 1e12)
+        # what the library dispatches, and the matrix rate of that
+        algo = (M.plan_block_f32(args.op, n, h, w, c, r, s_, k, bp) if args.blocked
+                else M.plan_f32(args.op, n, h, w, c, r, s_, k, M.Conv2DParams(*conv)))
+        split = M.plan_f32_split(args.op, n, h, w, c, r, s_, k, bp if args.blocked else M.Conv2DParams(*conv))
+        if split:
+            algo = "split " + algo
+        peak = PEAK_SPLIT_TFLOPS if split else PEAK_FP32_TFLOPS
+        t_mfma = flops / (peak * 1e12)
         t_hbm = nbytes / (PEAK_HBM_GBS * 1e9)
         bound = "mfma" if t_mfma >= t_hbm else "hbm"
         tf = flops / (ms * 1e-3) / 1e12
         gbs = nbytes / (ms * 1e-3) / 1e9
-        frac = tf / PEAK_FP32_TFLOPS if bound == "mfma" else gbs / PEAK_HBM_GBS
-        # what the library dispatches
-        algo = (M.plan_block_f32(args.op, n, h, w, c, r, s_, k, bp) if args.blocked
-                else M.plan_f32(args.op, n, h, w, c, r, s_, k, M.Conv2DParams(*conv)))
+        frac = tf / peak if bound == "mfma" else gbs / PEAK_HBM_GBS
         rows.append(dict(name=name, n=n, h=h, w=w, c=c, k=k, r=r, s=s_, groups=g, stride=sh, by=by, bx=bx, kernel=algo,
                          us=round(ms * 1e3, 2), tflops=round(tf, 3), gbs=round(gbs, 1), bound=bound,
-                         frac=round(frac, 4), verified=ok,
+                         peak=round(peak, 1), frac=round(frac, 4), verified=ok,
                          verified_on=("the image-0 problem vs the oracle; the full problem on small integers, AUTO "
                                       "== direct bit for bit" if args.op == "grad" else "image 0 vs the oracle")))
         del x, wt, y
@@ -395,10 +400,10 @@ def bench_fp32(args) -> None:
     if not rows:
         print(f"bench.py: unknown --fp32 shape {args.config}; known: {[c[0] for c in suite]}", file=sys.stderr)
         sys.exit(2)
-    print(f"{'shape':28s} {'kernel':11s} {'us':>10s} {'TFLOP/s':>8s} {'GB/s':>8s} {'bound':5s} {'frac':>6s} verified",
+    print(f"{'shape':28s} {'kernel':17s} {'us':>10s} {'TFLOP/s':>8s} {'GB/s':>8s} {'bound':5s} {'frac':>6s} verified",
           file=sys.stderr)
     for r in rows:
-        print(f"{r['name']:28s} {r['kernel']:11s} {r['us']:10.2f} {r['tflops']:8.2f} {r['gbs']:8.1f} {r['bound']:5s} "
+        print(f"{r['name']:28s} {r['kernel']:17s} {r['us']:10.2f} {r['tflops']:8.2f} {r['gbs']:8.1f} {r['bound']:5s} "
               f"{r['frac']:6.3f} {r['verified']}", file=sys.stderr)
     head = rows[0]
     suite_name = ("blocked bench suite (src/main.cpp:176-186)" if args.blocked
@@ -412,7 +417,7 @@ def bench_fp32(args) -> None:
                    "K": head["k"], "R": head["r"], "S": head["s"], "groups": head["groups"], "by": head["by"],
                    "bx": head["bx"], "kernel": head["kernel"], "timing": "eager back-to-back", "cache": "warm"},
         "roofline": {"bound": head["bound"], "achieved": head["tflops"] if head["bound"] == "mfma" else head["gbs"],
-                     "peak": PEAK_FP32_TFLOPS if head["bound"] == "mfma" else PEAK_HBM_GBS,
+                     "peak": head["peak"] if head["bound"] == "mfma" else PEAK_HBM_GBS,
                      "unit": "TFLOP/s" if head["bound"] == "mfma" else "GB/s", "frac": head["frac"], "traffic": None},
         "shapes": rows,
     }

@@ -381,8 +381,9 @@ int miq_block_grad_nhwc_f32(const float* x, const float* dy, float* dw, int32_t 
 typedef enum miq_f32_kernel {
   MIQ_F32_DIRECT = 0,          /* the reference CPU loop's order, one thread per output element (dx: per 4
                                   channels when (c/groups) % 4 == 0 and dx, w are 16-byte aligned) */
-  MIQ_F32_IGEMM = 1,           /* fp32 MFMA implicit GEMM, 128 pixels x 64 channels per workgroup */
-  MIQ_F32_IGEMM32 = 2,         /* the same with 256 pixels x 32 channels (groups of <= 32 channels) */
+  MIQ_F32_IGEMM = 1,           /* MFMA implicit GEMM: on split bf16 operands (miq_plan_f32_split), else fp32 MFMA with
+                                  128 pixels x 64 channels per workgroup */
+  MIQ_F32_IGEMM32 = 2,         /* the same for groups of <= 32 channels, the fp32 form with 256 pixels x 32 channels */
   MIQ_F32_DEPTHWISE = 3,       /* depthwise fprop or dx, 4 channels per thread */
   MIQ_F32_BPROP_IGEMM = 4,     /* stride-1 dx as the forward implicit GEMM over dy */
   MIQ_F32_GRAD_IGEMM = 5,      /* dw as a GEMM over pixels split across workgroups */
@@ -400,6 +401,18 @@ int miq_plan_f32(int32_t op, int32_t n, int32_t h, int32_t wdt, int32_t c, int32
  * miq_block_grad_nhwc_f32).  No reference counterpart. */
 int miq_plan_block_f32(int32_t op, int32_t n, int32_t h, int32_t wdt, int32_t c, int32_t r, int32_t s, int32_t k,
                        const miq_block_conv2d_params* p, int32_t algo, int32_t* kernel);
+
+/* Whether the MFMA form of an fp32 pass (op 0 fprop, 1 bprop, 2 grad, as AUTO and IGEMM run it)
+ * computes on operands split into three bf16 numbers each, and in which tile: tile[0] = 1, else
+ * every entry is 0 and the fp32 matrix instructions (or another kernel, miq_plan_f32) run.
+ * tile[1..3]: fprop, bprop: 16-position segments per wave, rows of waves, columns of waves (32
+ * channels each); grad: rows of waves (32 output channels each), columns of waves (input
+ * channels), wave groups that share a tile's positions.  tile[4..6]: images, rows and columns of
+ * a tile.  tile[7], tile[8]: fprop, bprop: 8-channel octets per chunk of the reduction, chunks;
+ * grad: tiles in flight in LDS, split partial sums.  p: block_by = block_bx = 1 for a plain
+ * filter.  16-byte aligned tensors; no GPU access.  No reference counterpart. */
+int miq_plan_f32_split(int32_t op, int32_t n, int32_t h, int32_t wdt, int32_t c, int32_t r, int32_t s, int32_t k,
+                       const miq_block_conv2d_params* p, int32_t tile[9]);
 
 /* ---- int32 batched matrix product -------------------------------------------------- */
 /* C[b] = op(A[b]) * op(B[b]) for b < batch, with int32 wrap-around (mod 2^32) products and

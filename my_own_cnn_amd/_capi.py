@@ -150,6 +150,7 @@ SIGNATURES = {
         C.c_int, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, C.POINTER(BlockConv2DParams), _I, _P]),
     "miq_block_grad_nhwc_f32": (
         C.c_int, [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, C.POINTER(BlockConv2DParams), _P, _I, _I, _P]),
+    "miq_plan_f32_split": (C.c_int, [_I, _I, _I, _I, _I, _I, _I, _I, C.POINTER(BlockConv2DParams), _PI]),
     "miq_plan_block_f32": (C.c_int, [_I, _I, _I, _I, _I, _I, _I, _I, C.POINTER(BlockConv2DParams), _I, _PI]),
 }
 

@@ -462,6 +462,20 @@ def plan_block_f32(op: str, n: int, h: int, w: int, c: int, r: int, s: int, k: i
     return F32_KERNEL_NAMES[out.value]
 
 
+def plan_f32_split(op: str, n: int, h: int, w: int, c: int, r: int, s: int, k: int,
+                   p=None) -> Optional[Tuple[int, ...]]:
+    """The tile (miq_plan_f32_split's tile[1..8]) in which an fp32 pass computes on split bf16
+    operands; None where it runs another kernel.  `p`: Conv2DParams, or BlockConv2DParams for the
+    blocked passes.  No GPU access."""
+    ops = {"fprop": 0, "bprop": 1, "grad": 2}
+    if op not in ops:
+        raise ValueError(f"op must be one of {sorted(ops)}, got {op!r}")
+    params = p if isinstance(p, BlockConv2DParams) else BlockConv2DParams(_as_params(p), 1, 1)
+    tile = (C.c_int32 * 9)()
+    check(lib().miq_plan_f32_split(ops[op], n, h, w, c, r, s, k, C.byref(params), tile), "plan_f32_split")
+    return tuple(tile[1:]) if tile[0] else None
+
+
 def conv2d_nhwc_f32(x, w, *, stride=1, padding=0, dilation=1, groups=1, algo="auto", out=None, stream=None):
     """fp32 convolution of device tensors: x (N, H, W, C), w (K, R, S, C/groups) -> (N, Ho, Wo, K)."""
     if x.dtype != torch.float32 or w.dtype != torch.float32:
@@ -516,7 +530,7 @@ def bmm_i32(a, b, *, trans_a=False, trans_b=False, out=None, stream=None):
 __all__ = [
     "bmm_i32", "bmm_matmul_i32", "conv2d_nhwc_f32", "launch_fprop_nhwc", "launch_bprop_nhwc", "launch_grad_nhwc",
     "launch_block_fprop_nhwc", "launch_block_bprop_nhwc", "launch_block_grad_nhwc", "plan_block_f32",
-    "DataType", "Conv2DParams", "BlockConv2DParams", "QParamsU8", "QParamsS5", "QConvDesc", "MiqError",
+    "plan_f32_split", "DataType", "Conv2DParams", "BlockConv2DParams", "QParamsU8", "QParamsS5", "QConvDesc", "MiqError",
     "qparams_array", "infer_conv_shape", "infer_block_conv_shape", "launch_fprop_nhwc_qi32",
     "launch_block_fprop_nhwc_qi32", "make_desc", "plan", "plan_f32", "qconv2d_nhwc_i8", "qconv2d_nhwc_i8_acc32",
     "qconv2d_nhwc_i8_dequant",

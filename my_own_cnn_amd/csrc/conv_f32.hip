@@ -1386,6 +1386,10 @@ size_t f32_grad_igemm_workspace(const Geom& g, const BlockGeom& bg) {
   return static_cast<size_t>(splits) * g.K * bg.By * bg.Bx * g.R * g.S * g.Cg * sizeof(float);
 }
 
+bool plan_f32_split_grad_igemm(const Geom& g, const BlockGeom& bg, int32_t* tile) {
+  return plan_f32_split_grad(g, bg, grad_max_splits(g, bg), tile);
+}
+
 hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw,
                                  float* ws, bool ordered, hipStream_t stream) {
   GradArgs a;
@@ -1655,6 +1659,10 @@ bool f32_bprop_igemm_eligible(const Geom& g, const BlockGeom& bg, const void* dy
 // Rows of the transposed filter are the original's input channels (b.Kg = g.Cg), its reduction
 // (r', s', ko < g.Kg = b.Cg); f32_igemm_launch takes ow_taps = R * S and ow_cg = b.Kg from b.
 // The filter blocks partition dy (bg: blocks of the original output).
+bool plan_f32_split_bprop(const Geom& g, const BlockGeom& bg, int32_t* tile) {
+  return plan_f32_split(f32_bprop_as_fprop(g), bg, true, tile);
+}
+
 hipError_t launch_f32_bprop_igemm(const Geom& g, const BlockGeom& bg, const float* dy, const float* w, float* dx,
                                   hipStream_t stream) {
   const Geom b = f32_bprop_as_fprop(g);

@@ -922,17 +922,41 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
   return best;
 }
 
+// The output regions: forward the filter blocks; blocked dx as many of the dx grid.
+void split_regions(const Geom& g, const BlockGeom& bg, bool transposed, int* rh, int* rw) {
+  const bool blocked_dx = transposed && bg.By * bg.Bx > 1;
+  *rh = blocked_dx ? (g.Ho + bg.By - 1) / bg.By : (transposed ? g.Ho : bg.bho);
+  *rw = blocked_dx ? (g.Wo + bg.Bx - 1) / bg.Bx : (transposed ? g.Wo : bg.bwo);
+}
+
+SplitPlan split_plan(const Geom& g, const BlockGeom& bg, bool transposed) {
+  int rh, rw;
+  split_regions(g, bg, transposed, &rh, &rw);
+  const int nreg = bg.By * bg.Bx;
+  SplitPlan p = transposed && nreg > 1 ? make_blocked_plan(g, bg, rh, rw) : make_plan(g, rh, rw, nreg, transposed);
+  if (p.variant >= 0 && (p.blocks <= 0 || p.blocks > (1LL << 22))) p.variant = -1;
+  return p;
+}
+
 }  // namespace
+
+bool plan_f32_split(const Geom& g, const BlockGeom& bg, bool transposed, int32_t* tile) {
+  const SplitPlan p = split_plan(g, bg, transposed);
+  if (p.variant < 0) return false;
+  const SplitVariant& v = kVariants[p.variant];
+  const int32_t out[8] = {v.nseg, v.wm, v.wn, p.ti, p.th, p.tw, p.co, p.nchunk};
+  std::copy(out, out + 8, tile);
+  return true;
+}
 
 bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                       int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err) {
   const int nreg = bg.By * bg.Bx;
   const bool blocked_dx = transposed && nreg > 1;
-  // the output regions: forward the filter blocks; blocked dx as many of the dx grid
-  const int rh = blocked_dx ? (g.Ho + bg.By - 1) / bg.By : (transposed ? g.Ho : bg.bho);
-  const int rw = blocked_dx ? (g.Wo + bg.Bx - 1) / bg.Bx : (transposed ? g.Wo : bg.bwo);
-  const SplitPlan p = blocked_dx ? make_blocked_plan(g, bg, rh, rw) : make_plan(g, rh, rw, nreg, transposed);
-  if (p.variant < 0 || p.blocks <= 0 || p.blocks > (1LL << 22)) return false;
+  const SplitPlan p = split_plan(g, bg, transposed);
+  if (p.variant < 0) return false;
+  int rh, rw;
+  split_regions(g, bg, transposed, &rh, &rw);
   SplitArgs a;
   a.x = x; a.w = w; a.bias = bias; a.y = y; a.g = g;
   a.kdim = g.R * g.S * g.Cg;

@@ -514,6 +514,15 @@ hipError_t launch_grad_shape(const SGradArgs& a, const SGradPlan& p, int taps, u
 
 }  // namespace
 
+bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, int32_t* tile) {
+  const SGradPlan p = grad_plan(g, bg, max_splits);
+  if (p.variant < 0) return false;
+  const GradVariant& v = kGradVariants[p.variant];
+  const int32_t out[8] = {v.wk, v.wc, v.wp, p.ti, p.th, p.tw, p.nbuf, static_cast<int32_t>(p.splits)};
+  std::copy(out, out + 8, tile);
+  return true;
+}
+
 bool launch_f32_split_grad(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw, float* ws,
                            long long max_splits, hipStream_t stream, long long* splits, hipError_t* err) {
   if (((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15u) != 0) return false;

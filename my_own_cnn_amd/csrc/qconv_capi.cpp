@@ -880,6 +880,27 @@ int miq_plan_block_f32(int32_t op, int32_t n, int32_t h, int32_t wdt, int32_t c,
   return plan_f32(op, g, bg, algo, kernel);
 }
 
+int miq_plan_f32_split(int32_t op, int32_t n, int32_t h, int32_t wdt, int32_t c, int32_t r, int32_t s, int32_t k,
+                       const miq_block_conv2d_params* p, int32_t tile[9]) {
+  if (tile == nullptr) return fail(MIQ_ERR_NULL_POINTER, "tile pointer is NULL");
+  std::fill(tile, tile + 9, 0);
+  miq::Geom g;
+  miq::BlockGeom bg;
+  int st = infer_block_geom(n, h, wdt, c, r, s, k, p, &g, &bg);
+  if (st != MIQ_OK) return st;
+  int32_t kernel = MIQ_F32_DIRECT;
+  st = plan_f32(op, g, bg, MIQ_ALGO_AUTO, &kernel);
+  if (st != MIQ_OK) return st;
+  switch (kernel) {
+    case MIQ_F32_IGEMM:
+    case MIQ_F32_IGEMM32: tile[0] = miq::plan_f32_split(g, bg, false, tile + 1); break;
+    case MIQ_F32_BPROP_IGEMM: tile[0] = miq::plan_f32_split_bprop(g, bg, tile + 1); break;
+    case MIQ_F32_GRAD_IGEMM: tile[0] = miq::plan_f32_split_grad_igemm(g, bg, tile + 1); break;
+    default: break;
+  }
+  return MIQ_OK;
+}
+
 int miq_bmm_i32(const int32_t* A, const int32_t* B, int32_t* C, int32_t batch, int32_t M, int32_t N, int32_t K,
                 int32_t trans_a, int32_t trans_b, void* stream) {
   if (batch < 0 || M < 0 || N < 0 || K < 0) return fail(MIQ_ERR_INVALID_ARGUMENT, "bmm extents must be >= 0");

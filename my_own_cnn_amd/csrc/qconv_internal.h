@@ -203,6 +203,8 @@ hipError_t launch_f32_igemm(const Geom& g, const BlockGeom& bg, const float* x, 
 // the blocks of the original output.  False when no tile of the shape fits (nothing is launched).
 bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                       int bias_mode, float* y, bool transposed, hipStream_t stream, hipError_t* err);
+// The tile that launch_f32_split takes, as miq_plan_f32_split's tile[1..8]; false where it takes none.
+bool plan_f32_split(const Geom& g, const BlockGeom& bg, bool transposed, int32_t* tile);
 hipError_t launch_f32_direct(const Geom& g, const BlockGeom& bg, const float* x, const float* w, const float* bias,
                              int bias_mode, float* y, hipStream_t stream);
 // fp32 depthwise (C/groups == K/groups == 1, C % 4 == 0, R*S*C <= 8192, 16-byte aligned x and y),
@@ -234,6 +236,12 @@ hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float
 // when the shape does not fit (nothing is launched).
 bool launch_f32_split_grad(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw, float* ws,
                            long long max_splits, hipStream_t stream, long long* splits, hipError_t* err);
+// The tile that launch_f32_split_grad takes with aligned tensors, as miq_plan_f32_split's
+// tile[1..8]; false where it takes none.
+bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, int32_t* tile);
+// The tiles of the two above as launch_f32_bprop_igemm and the ordered launch_f32_grad_igemm use them.
+bool plan_f32_split_bprop(const Geom& g, const BlockGeom& bg, int32_t* tile);
+bool plan_f32_split_grad_igemm(const Geom& g, const BlockGeom& bg, int32_t* tile);
 // Bias gradient of the blocked convolution: dbias (K * By * Bx floats, bias_mode 0 per block or
 // 1 shared) = the sum of dy over every output position of each block, in a fixed order, through
 // f32_block_dbias_workspace bytes of `ws` (nonzero for any non-empty dy).

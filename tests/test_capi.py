@@ -397,6 +397,28 @@ def test_plan_f32_names_the_kernel_each_pass_runs():
         M.plan_f32("fprop", 1, 2, 2, 16, 3, 3, 16, _capi.Conv2DParams(0, 0, 1, 1, 1, 1, 1))  # no output pixels
 
 
+def test_plan_f32_split_names_the_tile_of_the_split_kernels():
+    r50 = (32, 56, 56, 64, 3, 3, 64)
+    p1 = _capi.Conv2DParams(1, 1, 1, 1, 1, 1, 1)
+    b22 = M.BlockConv2DParams(p1, 2, 2)
+    for op in ("fprop", "bprop", "grad"):
+        for p in (p1, b22):
+            tile = M.plan_f32_split(op, *r50, p)
+            assert tile is not None and len(tile) == 8 and min(tile) >= 1, (op, tile)
+    # the fp32 instruction's and the other kernels' layers
+    assert M.plan_f32_split("fprop", 32, 56, 56, 64, 1, 1, 64) is None
+    assert M.plan_f32_split("bprop", *r50, _capi.Conv2DParams(1, 1, 2, 2, 1, 1, 1)) is None
+    assert M.plan_f32_split("grad", *r50, _capi.Conv2DParams(1, 1, 1, 1, 1, 1, 64)) is None
+    lib = M.lib()
+    tile = (C.c_int32 * 9)()
+    one = M.BlockConv2DParams(p1, 1, 1)
+    assert lib.miq_plan_f32_split(0, *r50, C.byref(one), None) == _capi.MIQ_ERR_NULL_POINTER
+    assert lib.miq_plan_f32_split(3, *r50, C.byref(one), tile) == _capi.MIQ_ERR_INVALID_ARGUMENT
+    assert lib.miq_plan_f32_split(0, *r50, None, tile) == _capi.MIQ_ERR_NULL_POINTER
+    with pytest.raises(ValueError, match="op"):
+        M.plan_f32_split("wgrad", *r50)
+
+
 def test_blocked_fp32_dropins_and_validation():
     # the reference's launch_block_{fprop,bprop,grad}_nhwc (conv_types.h:296-304), same mangled names
     syms = exported()

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 # (n, h, w, c, k, r, s, (ph, pw, sh, sw, dh, dw, groups))
 CASES = [
-    (1, 5, 4, 4, 33, 3, 3, (1, 1, 1, 1, 1, 1, 1)),       # one half octet, a channel past the tile
+    (1, 5, 4, 4, 33, 5, 5, (2, 2, 1, 1, 1, 1, 1)),       # one half octet, a channel past the tile
     (2, 17, 19, 12, 40, 3, 3, (1, 1, 1, 1, 1, 1, 1)),    # octet tail
     (3, 33, 29, 20, 48, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
     (5, 7, 7, 72, 65, 3, 3, (1, 1, 1, 1, 1, 1, 1)),      # several images per tile, an uneven chunk
@@ -31,7 +31,11 @@ CASES = [
     (24, 28, 28, 64, 96, 3, 3, (1, 1, 1, 1, 1, 1, 1)),   # enough tiles for the larger ones
     (32, 14, 14, 64, 256, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
     (40, 30, 26, 32, 32, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (32, 25, 20, 8, 36, 2, 3, (1, 1, 1, 1, 1, 1, 1)),    # one octet
+    (32, 66, 4, 96, 8, 2, 3, (1, 1, 1, 1, 1, 1, 1)),
+    (64, 23, 3, 64, 8, 3, 3, (1, 1, 1, 1, 2, 2, 1)),     # dx in the largest tile
 ]
+LAYOUTS = {(1, 4, 2), (2, 2, 2), (4, 2, 2), (4, 4, 1), (4, 4, 2)}  # segments, rows and columns of waves
 
 
 def conv64(x, w, conv):
@@ -50,6 +54,19 @@ def data(case, seed):
 def check(got, want, mag, kdim):
     err = (got.double() - want).abs()
     assert bool((err <= (kdim / 32 + 16) * 2.0 ** -23 * mag + 1e-300).all()), float((err / mag.clamp(min=1e-300)).max())
+
+
+def layout(op, n, h, w, c, k, r, s, conv, by=1, bx=1):
+    """The wave layout in which the pass computes on split operands, None where it does not."""
+    tile = M.plan_f32_split(op, n, h, w, c, r, s, k, M.BlockConv2DParams(M.Conv2DParams(*conv), by, bx))
+    return tile and tile[:3]
+
+
+def test_cases_reach_every_layout():
+    assert {layout("fprop", *c) for c in CASES} - {None} == LAYOUTS
+    assert {layout("bprop", *c) for c in CASES} - {None} == LAYOUTS
+    assert {layout("bprop", *c) for c in BLOCKED_DX} == LAYOUTS - {(1, 4, 2)}
+    assert len({c[1:] for c in GRADS_SPLIT}) == 8  # four layouts, one or two tiles in LDS
 
 
 @pytest.mark.parametrize("case", CASES, ids=[str(c) for c in CASES])
@@ -83,6 +100,7 @@ def test_empty_reductions_are_zero(device, taps):
 def test_blocked_forward(device, grid):
     n, h, w, c, k = 3, 16, 18, 40, 70
     by, bx = grid
+    assert layout("fprop", n, h, w, c, k, 3, 3, (1, 1, 1, 1, 1, 1, 1), by, bx)
     gen = torch.Generator().manual_seed(3)
     x, wt = torch.randn((n, h, w, c), generator=gen), torch.randn((k, by, bx, 3, 3, c), generator=gen)
     conv = (1, 1, 1, 1, 1, 1, 1)
@@ -185,17 +203,20 @@ def test_a_tiny_value_leaves_the_other_results(device, tiny):
     n, h, w, c, k = 2, 20, 20, 40, 72
     conv = (1, 1, 1, 1, 1, 1, 1)
     bp = M.BlockConv2DParams(M.Conv2DParams(*conv), 2, 2)
+    kd = 28  # output channels of dw: few enough for the split kernel at this size
+    assert layout("fprop", n, h, w, c, k, 3, 3, conv) and layout("bprop", n, h, w, c, k, 3, 3, conv)
+    assert layout("bprop", n, h, w, c, k, 3, 3, conv, 2, 2) and layout("grad", n, h, w, c, kd, 3, 3, conv)
     gen = torch.Generator().manual_seed(14)
     x, wt = torch.randn((n, h, w, c), generator=gen), torch.randn((k, 3, 3, c), generator=gen)
     dy, wb = torch.randn((n, h, w, k), generator=gen), torch.randn((k, 2, 2, 3, 3, c), generator=gen)
 
     def outputs(x, wt, dy):
         x, wt, dy = x.to(device), wt.to(device), dy.to(device)
-        y, dx, dxb, dw = torch.empty_like(dy), torch.empty_like(x), torch.empty_like(x), torch.empty_like(wt)
+        y, dx, dxb, dw = torch.empty_like(dy), torch.empty_like(x), torch.empty_like(x), torch.empty_like(wt[:kd])
         M.launch_fprop_nhwc(x, wt, y, n, h, w, c, 3, 3, k, conv)
         M.launch_bprop_nhwc(dy, wt, dx, n, h, w, c, 3, 3, k, conv)
         M.launch_block_bprop_nhwc(dy, wb.to(device), dxb, n, h, w, c, 3, 3, k, bp)
-        M.launch_grad_nhwc(x, dy, dw, n, h, w, c, 3, 3, k, conv)
+        M.launch_grad_nhwc(x, dy[..., :kd].contiguous(), dw, n, h, w, c, 3, 3, kd, conv)
         return y.cpu(), dx.cpu(), dxb.cpu(), dw.cpu()
 
     def put(t, at, v):
@@ -224,11 +245,15 @@ def test_subnormal_products(device, exp):
     x, wt = data((n, h, w, c, k, 3, 3, conv), 16)
     dy = torch.randn((n, h, w, k), generator=torch.Generator().manual_seed(17))
     x, wt, dy = x * 2.0 ** exp, wt * 2.0 ** exp, dy * 2.0 ** exp
-    y, dx, dw = (torch.full(t.shape, 7.0, device=device) for t in (dy, x, wt))
-    dims = (n, h, w, c, 3, 3, k, conv)
-    M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims)
-    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims)
-    M.launch_grad_nhwc(x.to(device), dy.to(device), dw, *dims)
+    kd = 32  # output channels of dw: few enough for the split kernel at this size
+    dyd = dy[..., :kd].contiguous()
+    assert layout("fprop", n, h, w, c, k, 3, 3, conv) and layout("bprop", n, h, w, c, k, 3, 3, conv)
+    assert layout("grad", n, h, w, c, kd, 3, 3, conv)
+    y, dx, dw = (torch.full(t.shape, 7.0, device=device) for t in (dy, x, wt[:kd]))
+    dims = (n, h, w, c, 3, 3)
+    M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims, k, conv)
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims, k, conv)
+    M.launch_grad_nhwc(x.to(device), dyd.to(device), dw, *dims, kd, conv)
     xg = x.double().requires_grad_()
     want_dx, = torch.autograd.grad(conv64(xg, wt, conv), xg, dy.double())
     mag_dx, = torch.autograd.grad(conv64(xg, wt.abs(), conv), xg, dy.double().abs())
@@ -236,18 +261,18 @@ def test_subnormal_products(device, exp):
     for got, want, mag, kdim, roundings in (
             (y, conv64(x, wt, conv), conv64(x.abs(), wt.abs(), conv), 9 * c, 1),
             (dx, want_dx, mag_dx, 9 * k, 1),
-            (dw, grad_want(x, dy, wt.shape, conv), grad_want(x, dy, wt.shape, conv, torch.abs), n * h * w + 512, parts)):
+            (dw, grad_want(x, dyd, dw.shape, conv), grad_want(x, dyd, dw.shape, conv, torch.abs), n * h * w + 512, parts)):
         err = (got.cpu().double() - want).abs()
         assert bool((err <= (kdim / 32 + 16) * 2.0 ** -23 * mag + roundings * 2.0 ** -150).all()), float(err.max())
 
 
-# filter gradients: (n, h, w, c, k, r, s, conv); channel counts on both sides of the wave layouts
+# filter gradients of small layers, most of which the fp32 GEMM takes: (n, h, w, c, k, r, s, conv)
 GRADS = [
     (2, 9, 11, 4, 8, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
     (3, 19, 17, 36, 68, 3, 3, (1, 1, 1, 1, 1, 1, 1)),     # channels past the tiles
     (9, 7, 7, 64, 96, 3, 3, (1, 1, 1, 1, 1, 1, 1)),       # several images per tile
-    (2, 31, 29, 32, 32, 3, 3, (1, 1, 2, 2, 1, 1, 1)),     # stride, four wave groups
-    (1, 26, 40, 68, 28, 3, 3, (2, 0, 1, 2, 2, 1, 1)),     # dilation, two wave groups
+    (2, 31, 29, 32, 32, 3, 3, (1, 1, 2, 2, 1, 1, 1)),     # stride
+    (1, 26, 40, 68, 28, 3, 3, (2, 0, 1, 2, 2, 1, 1)),     # dilation
     (2, 21, 18, 20, 72, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
     (2, 15, 14, 128, 64, 1, 1, (0, 0, 1, 1, 1, 1, 1)),    # one tap, two channel tiles per wave
     (2, 13, 15, 16, 40, 2, 3, (1, 1, 1, 1, 1, 1, 1)),     # fewer taps than a workgroup takes
@@ -257,15 +282,45 @@ GRADS = [
 ]
 
 
+# filter gradients on split operands: the case, its wave layout (32-channel rows, columns of input
+# channels, wave groups that share a tile's positions) and the tiles in flight in LDS
+GRADS_SPLIT = [
+    ((1, 14, 21, 68, 36, 1, 1, (0, 0, 1, 1, 1, 1, 1)), (2, 4, 1), 2),      # one tap, two channel tiles per wave
+    ((3, 71, 26, 36, 68, 3, 3, (0, 1, 1, 1, 1, 1, 1)), (2, 4, 1), 2),
+    ((3, 114, 63, 36, 68, 3, 3, (1, 1, 2, 2, 1, 1, 1)), (2, 4, 1), 2),     # stride
+    ((5, 71, 68, 36, 68, 3, 3, (1, 1, 2, 2, 2, 3, 1)), (2, 4, 1), 1),      # stride and dilation
+    ((9, 40, 29, 36, 68, 3, 4, (1, 2, 1, 2, 2, 3, 1)), (2, 4, 1), 1),      # 12 taps: two workgroups' worth
+    ((1, 52, 50, 64, 64, 5, 5, (2, 2, 1, 1, 1, 1, 1)), (2, 4, 1), 2),
+    ((1, 17, 23, 20, 40, 1, 1, (0, 0, 1, 1, 1, 1, 1)), (2, 2, 2), 2),      # one tap, one channel tile
+    ((5, 84, 45, 20, 40, 3, 3, (0, 1, 1, 1, 2, 3, 1)), (2, 2, 2), 2),
+    ((2, 78, 111, 40, 80, 3, 3, (1, 1, 1, 2, 2, 3, 2)), (2, 2, 2), 2),     # groups
+    ((5, 125, 114, 20, 40, 3, 3, (1, 1, 2, 2, 1, 1, 1)), (2, 2, 2), 1),
+    ((9, 23, 50, 20, 40, 5, 5, (0, 2, 1, 1, 1, 1, 1)), (2, 2, 2), 1),
+    ((2, 114, 44, 68, 28, 1, 1, (0, 0, 1, 2, 1, 1, 1)), (1, 4, 2), 1),
+    ((1, 9, 38, 40, 12, 3, 3, (1, 1, 1, 1, 1, 1, 1)), (1, 4, 2), 2),
+    ((2, 89, 48, 40, 12, 3, 3, (1, 1, 2, 1, 2, 1, 1)), (1, 4, 2), 1),
+    ((5, 23, 11, 68, 28, 2, 3, (0, 1, 1, 1, 1, 1, 1)), (1, 4, 2), 1),      # fewer taps than a workgroup takes
+    ((1, 35, 9, 20, 28, 3, 3, (0, 1, 1, 1, 2, 3, 1)), (1, 2, 4), 2),
+    ((2, 96, 94, 32, 32, 3, 3, (1, 1, 2, 2, 1, 1, 1)), (1, 2, 4), 2),
+    ((2, 51, 82, 16, 24, 3, 3, (1, 1, 2, 1, 2, 1, 1)), (1, 2, 4), 1),
+    ((1, 128, 10, 16, 24, 2, 3, (0, 1, 1, 1, 2, 3, 1)), (1, 2, 4), 1),
+]
+
+
 def grad_want(x, dy, wshape, conv, f=lambda v: v):
     w = torch.zeros(wshape, dtype=torch.float64, requires_grad=True)
     return torch.autograd.grad(conv64(f(x), w, conv), w, f(dy).double())[0]
 
 
-@pytest.mark.parametrize("case", GRADS, ids=[str(c) for c in GRADS])
+@pytest.mark.parametrize("case", GRADS + GRADS_SPLIT, ids=str)
 def test_filter_gradient(device, case):
+    seed = 31 + (GRADS + GRADS_SPLIT).index(case)
+    if len(case) == 3:
+        case, waves, tiles = case
+        plan = M.plan_f32_split("grad", *case[:4], *case[5:7], case[4], case[7])
+        assert plan and (plan[:3], plan[6]) == (waves, tiles), plan
     n, h, w, c, k, r, s, conv = case
-    x, wt = data(case, 31 + GRADS.index(case))
+    x, wt = data(case, seed)
     dy = torch.randn(conv64(x, wt, conv).shape, generator=torch.Generator().manual_seed(4))
     dw = torch.full(wt.shape, 7.0, device=device)
     M.launch_grad_nhwc(x.to(device), dy.to(device), dw, n, h, w, c, r, s, k, conv)
@@ -273,7 +328,7 @@ def test_filter_gradient(device, case):
     check(dw.cpu(), grad_want(x, dy, wt.shape, conv), grad_want(x, dy, wt.shape, conv, torch.abs), dy[..., 0].numel() + 512)
 
 
-@pytest.mark.parametrize("shape", [(8, 40, 40, 64, 64), (8, 40, 40, 32, 32), (2, 40, 40, 96, 40)])
+@pytest.mark.parametrize("shape", [(8, 40, 40, 64, 64), (8, 40, 40, 32, 32), (4, 40, 40, 96, 40)])
 def test_errors_do_not_lean(device, shape):
     """The errors of a result's elements cancel: their mean is a small part of their rms.  The sums of
     the matrix core alone lean one way (means of 0.3 rms forward, 0.8 in the filter gradient).  Over
@@ -285,6 +340,8 @@ def test_errors_do_not_lean(device, shape):
     x, wt = torch.randn((n, h, w, c), generator=gen).clamp(min=0), torch.randn((k, 3, 3, c), generator=gen)
     dy, wb = torch.randn((n, h, w, k), generator=gen), torch.randn((k, 2, 2, 3, 3, c), generator=gen)
     dims = (n, h, w, c, 3, 3, k)
+    for op, b in (("fprop", 1), ("bprop", 1), ("bprop", 2), ("grad", 1)):
+        assert layout(op, n, h, w, c, k, 3, 3, conv, b, b), op
     y, dx, dxb, dw = (torch.empty(t.shape, device=device) for t in (dy, x, x, wt))
     M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims, conv)
     M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims, conv)
@@ -300,12 +357,13 @@ def test_errors_do_not_lean(device, shape):
 
 @pytest.mark.parametrize("grid", [(2, 3), (4, 1)])
 def test_blocked_filter_gradient(device, grid):
-    n, h, w, c, k = 5, 16, 18, 40, 70
+    n, h, w, c, k = 21, 16, 18, 40, 70
     by, bx = grid
     gen = torch.Generator().manual_seed(8)
     x, dy = torch.randn((n, h, w, c), generator=gen), torch.randn((n, h, w, k + 2), generator=gen)
     k += 2
     conv = (1, 1, 1, 1, 1, 1, 1)
+    assert layout("grad", n, h, w, c, k, 3, 3, conv, by, bx)
     dw = torch.empty((k, by, bx, 3, 3, c), device=device)
     M.launch_block_grad_nhwc(x.to(device), dy.to(device), dw, n, h, w, c, 3, 3, k,
                              M.BlockConv2DParams(M.Conv2DParams(*conv), by, bx))
@@ -318,10 +376,11 @@ def test_blocked_filter_gradient(device, grid):
             check(got[:, i, j], grad_want(x, d, (k, 3, 3, c), conv), grad_want(x, d, (k, 3, 3, c), conv, torch.abs), n * h * w)
 
 
-@pytest.mark.parametrize("shape", [(2, 24, 24, 64, 64), (2, 24, 24, 32, 32)])
+@pytest.mark.parametrize("shape", [(12, 24, 24, 64, 64), (2, 24, 24, 32, 32)])
 def test_filter_gradient_of_special_values(device, shape):
     n, h, w, c, k = shape
     conv = (1, 1, 1, 1, 1, 1, 1)
+    assert layout("grad", n, h, w, c, k, 3, 3, conv)
     gen = torch.Generator().manual_seed(9)
     x, dy = torch.randn((n, h, w, c), generator=gen), torch.randn((n, h, w, k), generator=gen)
     args = (n, h, w, c, 3, 3, k, conv)

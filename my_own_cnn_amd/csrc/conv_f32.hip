@@ -1248,13 +1248,13 @@ __global__ void __launch_bounds__(kDirectThreads) f32_dbias_part_kernel(const fl
   const int np = min(P - p0, kDbiasChunk);
   const int rc = bg.bho * bg.bwo;
   const float* dyk = dy + min(k, g.K - 1);
-  // wave w copies positions kPer w .. of the run; those past its end repeat the last position
-  // and are not added
+  // wave w copies positions kPer w .. of the run, 16 at a time; those past its end within a 16
+  // repeat the last position and are not added
   int p = p0 + min(wave * kPer, np - 1);
   int n = p / rc;
   int lho = (p - n * rc) / bg.bwo;
   int lwo = p - n * rc - lho * bg.bwo;
-  for (int j0 = 0; j0 < kPer; j0 += 16) {
+  for (int j0 = 0; j0 < kPer && wave * kPer + j0 < np; j0 += 16) {  // uniform
     float v[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {

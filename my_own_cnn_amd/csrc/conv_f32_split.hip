@@ -890,14 +890,72 @@ hipError_t launch_split(const SplitArgs& a, const SplitPlan& p, hipStream_t stre
 
 namespace {
 
+// Along one dimension, the worst window of `len` output positions at multiples of `step` inside a
+// region of `rlen`: how many filter blocks (of `blk` input positions) its taps reach, and the taps
+// summed over them.  Regions 0 and 1 stand for all: an inner region has neighbours on both sides.
+struct Reach1 {
+  int taps, blocks;
+};
+Reach1 worst_reach(int in, int nreg, int rlen, int step, int len, int blk, int R, int d, int pad) {
+  Reach1 worst{0, 0};
+  for (int q = 0; q < std::min(nreg, 2); ++q)
+    for (int o = 0; o < rlen; o += step) {
+      const int lo = q * rlen + o - pad, hi = lo + len - 1;  // the window on the input, tap 0
+      const int y1 = std::min(hi + (R - 1) * d, in - 1);
+      Reach1 now{0, 0};
+      for (int y = std::max(lo, 0) / blk * blk; y <= y1; y += blk) {
+        const int r0 = y > hi ? (y - hi + d - 1) / d : 0;
+        const int r1 = std::min(R - 1, (std::min(y + blk, in) - 1 - lo) / d);
+        if (r1 < r0) continue;
+        now.taps += r1 - r0 + 1;
+        ++now.blocks;
+      }
+      if (now.taps > worst.taps) worst = now;
+    }
+  return worst;
+}
+
+// Estimated microseconds of the blocked dx: both kernels wait for their worst tile, whose pieces
+// (stages of the split kernel, 16-channel chunks of the fp32 GEMM) pass one after the other.  Fitted to
+// 422 layers of 1 x 2 to 4 x 4 blocks, 1 to 32 images, 3x3 and 5x5 taps: the GEMM within 4% on
+// average, the split within 11%.
+double split_blocked_us(const Geom& g, const BlockGeom& bg, int rh, int rw, const SplitPlan& p) {
+  const Reach1 a = worst_reach(g.H, bg.By, rh, p.th, p.th, bg.bho, g.R, g.dh, g.ph);
+  const Reach1 b = worst_reach(g.W, bg.Bx, rw, p.tw, p.tw, bg.bwo, g.S, g.dw, g.pw);
+  const double so = std::max(4, 2 * kVariants[p.variant].wm);
+  const double stages = p.nchunk * (static_cast<double>(a.taps) * b.taps * p.co / so + 0.5 * a.blocks * b.blocks);
+  constexpr double fit[4][3] = {{5.5, 1.23, 9.1}, {8.3, 0.95, 3.9}, {6.2, 0.68, 8.9}, {3.0, 1.35, 6.4}};
+  const double* f = fit[p.variant];
+  return f[0] + f[1] * stages * std::max(1.0, p.blocks / 256.0) + f[2] * p.nchunk;
+}
+double igemm_blocked_us(const Geom& g, const BlockGeom& bg, int rh, int rw) {
+  const int bm = g.Kg <= 32 ? 256 : 128, bn = g.Kg <= 32 ? 32 : 64;
+  // its tile: bm (position, image) pairs, the image fastest; whole columns where it wraps a row
+  const int pos = (bm + g.N - 1) / g.N;
+  const bool in_row = bm % g.N == 0 && rw % pos == 0;
+  const int rows = in_row ? 1 : std::min(rh, (pos + rw - 2) / rw + 1);
+  const Reach1 a = worst_reach(g.H, bg.By, rh, 1, rows, bg.bho, g.R, g.dh, g.ph);
+  const Reach1 b = in_row ? worst_reach(g.W, bg.Bx, rw, pos, pos, bg.bwo, g.S, g.dw, g.pw)
+                          : worst_reach(g.W, bg.Bx, rw, rw, rw, bg.bwo, g.S, g.dw, g.pw);
+  const double chunks = static_cast<double>(a.taps) * b.taps * g.Cg / 16;
+  const double tiles = std::ceil(static_cast<double>(g.N) * rh * rw / bm) * bg.By * bg.Bx * ((g.Kg + bn - 1) / bn) * g.G;
+  return 12.1 + 0.832 * chunks * std::max(1.0, tiles / 256);
+}
+
 // Blocked dx: 16 images (or all of fewer) x a few positions per tile, tiles inside regions of
-// ceil(Ho / By) x ceil(Wo / Bx), so that most reach one filter block.
+// ceil(Ho / By) x ceil(Wo / Bx), so that most reach one filter block.  Variant -1 where the fp32
+// implicit GEMM is the faster kernel: by the two estimates (32 x 14 x 14, 128 -> 64 5x5 in 2 x 2
+// blocks 156 us against 215; over 499 layers no call more than 1.11 times the faster kernel's time
+// but one, where the split alone was up to 1.42), and with one tap unless a filter block serves at
+// most 32 positions: few stages, all latency (16 x 16 x 16, 128 -> 256 in 4 x 4 blocks 20 against 43 us;
+// 512 -> 512 mostly slower, 35 against 48, at best 106 against 90; 16 positions a block 19 against 17).
 SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) {
   SplitPlan best{};
   best.variant = -1;
   const long long nreg = static_cast<long long>(bg.By) * bg.Bx;
   if (!plain_extents(g) || g.dh <= 0 || g.dw <= 0 || g.R > 16 || g.S > 16) return best;
-  if (g.R * g.S == 1 && g.Cg < 128) return best;
+  const bool one_tap = g.R * g.S == 1;
+  if (one_tap && (g.Cg < 128 || static_cast<long long>(g.N) * bg.bho * bg.bwo > 32)) return best;
   if (static_cast<double>(g.Kg) * nreg * g.R * g.S * g.Cg * 4 >= 2147483647.0) return best;
   for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
     if ((kVariants[v].wn == 1) != (g.Kg <= 32) || kVariants[v].nseg == 1) continue;
@@ -919,6 +977,10 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
       }
     }
   }
+  // more than 9 taps on full tiles of 16 images take up to 1.7 times their estimate
+  const double margin = g.R * g.S <= 9 ? 1.0 : 0.75;
+  if (best.variant >= 0 && !one_tap &&
+      split_blocked_us(g, bg, rh, rw, best) > margin * igemm_blocked_us(g, bg, rh, rw)) best.variant = -1;
   return best;
 }
 

@@ -42,6 +42,8 @@ EDGE = [
     ("5x5_dil2_b3x3", 1, 18, 18, 16, 40, 5, 5, (4, 4, 1, 1, 2, 2, 1), 3, 3),
     ("tiny_blocks_1x1_each", 2, 8, 8, 8, 16, 3, 3, (1, 1, 1, 1, 1, 1, 1), 8, 8),
     ("kg_gt_64_tiles", 1, 10, 12, 32, 136, 3, 3, (1, 1, 1, 1, 1, 1, 1), 2, 3),
+    ("pointwise_64_b2x2", 3, 14, 18, 64, 64, 1, 1, (0, 0, 1, 1, 1, 1, 1), 2, 2),    # one tap: dx on the fp32
+    ("pointwise_72_100_b4x4", 2, 12, 20, 72, 100, 1, 1, (0, 0, 1, 1, 1, 1, 1), 4, 4),  # GEMM, 64 channels a tile
 ]
 CASES = SUITE + EDGE
 IDS = [c[0] for c in CASES]
@@ -169,6 +171,9 @@ def test_block_plan_and_dispatch(device):
     assert M.plan_block_f32("fprop", n, h, w, c, r, s, k, p) == "igemm"
     assert M.plan_block_f32("bprop", n, h, w, c, r, s, k, p) == "bprop_igemm"
     assert M.plan_block_f32("grad", n, h, w, c, r, s, k, p) == "grad_igemm"
+    for e in EDGE[-2:]:
+        assert M.plan_block_f32("bprop", *_dims(e)[:4], e[6], e[7], e[5], _params(e)) == "bprop_igemm"
+        assert M.plan_f32_split("bprop", *_dims(e)[:4], e[6], e[7], e[5], _params(e)) is None
     e = EDGE[0]  # stride 2: dx has no MFMA form
     assert M.plan_block_f32("bprop", *_dims(e)[:4], e[6], e[7], e[5], _params(e)) == "direct"
     with pytest.raises(M.MiqError, match="stride 1"):

@@ -65,7 +65,8 @@ def layout(op, n, h, w, c, k, r, s, conv, by=1, bx=1):
 def test_cases_reach_every_layout():
     assert {layout("fprop", *c) for c in CASES} - {None} == LAYOUTS
     assert {layout("bprop", *c) for c in CASES} - {None} == LAYOUTS
-    assert {layout("bprop", *c) for c in BLOCKED_DX} == LAYOUTS - {(1, 4, 2)}
+    assert {layout("bprop", *c) for c in BLOCKED_DX} - {None} == LAYOUTS - {(1, 4, 2)}
+    assert [layout("bprop", *c) is None for c in BLOCKED_DX if c[5] * c[6] == 1] == [True, False]
     assert len({c[1:] for c in GRADS_SPLIT}) == 8  # four layouts, one or two tiles in LDS
 
 
@@ -139,7 +140,9 @@ BLOCKED_DX = [
     (17, 12, 12, 24, 16, 5, 5, (2, 2, 1, 1, 1, 1, 1), 6, 4),
     (2, 14, 15, 48, 40, 3, 3, (2, 0, 1, 1, 2, 1, 1), 2, 1),
     (16, 10, 9, 64, 128, 3, 2, (0, 1, 1, 1, 1, 1, 2), 4, 2),
-    (33, 8, 8, 40, 160, 1, 1, (0, 0, 1, 1, 1, 1, 1), 2, 2),
+    (33, 8, 8, 40, 160, 1, 1, (0, 0, 1, 1, 1, 1, 1), 2, 2),  # one tap: the fp32 implicit GEMM
+    (2, 8, 8, 40, 160, 1, 1, (0, 0, 1, 1, 1, 1, 1), 2, 2),   # but for at most 32 positions a block
+    (20, 10, 6, 48, 16, 1, 3, (0, 1, 1, 1, 1, 1, 1), 1, 2),
 ]
 
 

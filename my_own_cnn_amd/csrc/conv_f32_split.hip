@@ -822,6 +822,20 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
   }
 }
 
+// One tap: whether the split is the faster kernel in the chosen tile (us, fp32 GEMM against split).
+// Each stage is as long as the latency of its filter values, so it has to hold 8 octets: tiles of 4
+// waves hold 4 a stage (1x1 32 x 14 x 14, 256 -> 64 15.8 / 17.0, until 512 channels: 8 x 14 x 14,
+// 128 -> 512 dx 30.2 / 27.1), and 256 positions leave room for fewer than 8 octets of halo (112 x 112,
+// 256 -> 16 17.8 / 22.4; dx over more than 256 workgroups 33.0 / 29.1).  A last round of few workgroups
+// is a whole one (8 x 72 x 72, 96 -> 128 dx in 352: 25.3 / 28.0).  Of 803 layers no call is more than 1.12
+// times the faster kernel's time, where the split alone was up to 1.27 (blocked forward, 256 -> 32).
+bool one_tap_pays(const Geom& g, const SplitPlan& p, bool transposed) {
+  const SplitVariant& v = kVariants[p.variant];
+  if (v.wm < 4) return g.Cg >= 512;
+  if (v.wn == 1) return p.nchunk * p.nst <= (g.Cg + 63) / 64 || (transposed && p.blocks > 256);
+  return v.nseg == 1 || p.blocks <= 256 || 256.0 * ((p.blocks + 255) / 256) <= 1.35 * static_cast<double>(p.blocks);
+}
+
 // The tile of a launch, or variant -1 where the fp32 implicit GEMM is the faster kernel (measured
 // on a 32 x 56 x 56 layer unless a size is given): with one tap nothing is read twice from the
 // halo and a short reduction leaves the split unpaid (1x1 128 -> 256: 100 against 89 us; 512 -> 128
@@ -858,6 +872,7 @@ SplitPlan make_plan(const Geom& g, int rh, int rw, long long nreg, bool transpos
       if (tw <= 8) break;
     }
   }
+  if (best.variant >= 0 && g.R * g.S == 1 && !one_tap_pays(g, best, transposed)) best.variant = -1;
   return best;
 }
 

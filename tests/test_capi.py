@@ -419,6 +419,38 @@ def test_plan_f32_split_names_the_tile_of_the_split_kernels():
         M.plan_f32_split("wgrad", *r50)
 
 
+# (op, (n, h, w, c, r, s, k), blocks, whether the pass computes on split operands)
+SPLIT_ROUTES = [
+    ("fprop", (1, 56, 56, 256, 1, 1, 64), 1, True),
+    ("fprop", (32, 14, 14, 256, 1, 1, 64), 1, False),   # 4 waves a tile, 4 octets a stage
+    ("fprop", (1, 112, 112, 256, 1, 1, 16), 1, False),  # 256 positions, fewer than 8 octets of halo
+    ("fprop", (8, 16, 16, 256, 1, 1, 32), 2, False),
+    ("fprop", (32, 56, 56, 256, 1, 1, 128), 1, True),
+    ("bprop", (8, 14, 14, 128, 1, 1, 512), 1, True),    # 4 waves, but 512 channels
+    ("bprop", (8, 72, 72, 96, 1, 1, 128), 1, False),    # a round and a third
+    ("bprop", (16, 16, 16, 128, 1, 1, 256), 4, False),  # blocked, one tap
+    ("bprop", (1, 16, 16, 128, 1, 1, 256), 4, True),    # 16 positions a block
+    ("bprop", (32, 14, 14, 128, 5, 5, 64), 2, False),   # 16 images, 25 taps
+    ("bprop", (1, 14, 14, 128, 5, 5, 64), 2, True),
+    ("bprop", (32, 56, 56, 64, 3, 3, 64), 4, True),
+    ("grad", (1, 7, 7, 64, 5, 5, 64), 1, False),        # at most one workgroup of the GEMM per CU
+    ("grad", (8, 28, 28, 64, 3, 3, 64), 1, False),
+    ("grad", (8, 28, 28, 128, 3, 3, 128), 1, True),
+    ("grad", (4, 14, 14, 16, 3, 3, 16), 1, True),       # few taps, half a tile of output channels
+    ("grad", (1, 7, 7, 16, 3, 3, 16), 1, False),
+    ("grad", (1, 7, 7, 128, 1, 1, 128), 1, True),
+    ("grad", (1, 8, 8, 32, 3, 3, 64), 4, False),
+    ("grad", (16, 16, 16, 128, 3, 3, 256), 4, True),
+]
+
+
+@pytest.mark.parametrize("op,dims,blocks,split", SPLIT_ROUTES)
+def test_fp32_passes_run_on_split_operands_where_they_are_faster(op, dims, blocks, split):
+    pad = dims[4] // 2
+    p = M.BlockConv2DParams(_capi.Conv2DParams(pad, pad, 1, 1, 1, 1, 1), blocks, blocks)
+    assert (M.plan_f32_split(op, *dims, p) is not None) == split
+
+
 def test_blocked_fp32_dropins_and_validation():
     # the reference's launch_block_{fprop,bprop,grad}_nhwc (conv_types.h:296-304), same mangled names
     syms = exported()

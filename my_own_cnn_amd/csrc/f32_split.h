@@ -22,9 +22,10 @@ struct Split8 {
 };
 
 // Eight fp32 values times `scale` as three bf16 each.  With a scale of 2^23 every fp32 value below
-// 2^105 is carried exactly, subnormals among them: a residual of the scaled value is a multiple of
+// 2^104 is carried exactly, subnormals among them: a residual of the scaled value is a multiple of
 // 2^-126, so each piece is zero or a normal bf16, and the corrections of a product that fp32 holds
-// stay above the subnormal range.  A larger value becomes infinite, and whatever it reaches infinite or NaN.
+// stay above the subnormal range.  From about 2^105 a value becomes infinite, and whatever it reaches infinite
+// or NaN.
 __device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, float scale) {
   Split8 out;
 #pragma unroll

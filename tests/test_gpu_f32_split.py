@@ -2,8 +2,10 @@
 stages and chunks, and the inputs that it hands back to the fp32 instructions.
 
 Bound against 64 bits: a K-block of 32 reduction values is summed with a few fp32 roundings of
-its own and added with one more, and the dropped products are below 2^-26 of each term, so every
-output is within (K / 32 + 16) 2^-23 of the sum of |x w| (a factor two in hand)."""
+its own (of up to 2^-23 each, the matrix core rounds down) and added with one of 2^-24 more, and the
+dropped products are at most 2^-24 of each term, so every output is within (K / 32 + 16) 2^-23 of the
+sum of |x w|: K / 32 times 2^-24 for the additions, and less than 16 times 2^-23 for a K-block's own
+roundings, the dropped products and the scale (a factor two in hand)."""
 import numpy as np
 import pytest
 import torch
@@ -267,6 +269,38 @@ def test_subnormal_products(device, exp):
             (dw, grad_want(x, dyd, dw.shape, conv), grad_want(x, dyd, dw.shape, conv, torch.abs), n * h * w + 512, parts)):
         err = (got.cpu().double() - want).abs()
         assert bool((err <= (kdim / 32 + 16) * 2.0 ** -23 * mag + roundings * 2.0 ** -150).all()), float(err.max())
+
+
+@pytest.mark.parametrize("signs", [False, True])
+def test_operands_with_the_largest_dropped_products(device, signs):
+    """1 + 2^-8 - 2^-17 splits into 1, 2^-8 and -2^-17: the dropped products of every term are 2^-24.01
+    of it, all one way.  Every result is within 2^-24 of the sum of |x w| for them and as much for the
+    roundings, which are few: the terms are equal, so that short sums of them are nearly exact."""
+    n, h, w, c, k = 2, 24, 24, 32, 64
+    conv = (1, 1, 1, 1, 1, 1, 1)
+    value = 1 + 2.0 ** -8 - 2.0 ** -17
+    gen = torch.Generator().manual_seed(19)
+
+    def fill(*shape):
+        return value * (torch.randint(0, 2, shape, generator=gen) * 2.0 - 1 if signs else torch.ones(shape))
+
+    x, wt, dy = fill(n, h, w, c), fill(k, 3, 3, c), fill(n, h, w, k)
+    kd = 32  # output channels of dw: few enough for the split kernel at this size
+    dyd = dy[..., :kd].contiguous()
+    assert layout("fprop", n, h, w, c, k, 3, 3, conv) and layout("bprop", n, h, w, c, k, 3, 3, conv)
+    assert layout("grad", n, h, w, c, kd, 3, 3, conv)
+    y, dx, dw = (torch.full(t.shape, 7.0, device=device) for t in (dy, x, wt[:kd]))
+    dims = (n, h, w, c, 3, 3)
+    M.launch_fprop_nhwc(x.to(device), wt.to(device), y, *dims, k, conv)
+    M.launch_bprop_nhwc(dy.to(device), wt.to(device), dx, *dims, k, conv)
+    M.launch_grad_nhwc(x.to(device), dyd.to(device), dw, *dims, kd, conv)
+    xg = x.double().requires_grad_()
+    want_dx, = torch.autograd.grad(conv64(xg, wt, conv), xg, dy.double())
+    mag_dx, = torch.autograd.grad(conv64(xg, wt.abs(), conv), xg, dy.double().abs())
+    for got, want, mag in ((y, conv64(x, wt, conv), conv64(x.abs(), wt.abs(), conv)), (dx, want_dx, mag_dx),
+                           (dw, grad_want(x, dyd, dw.shape, conv), grad_want(x, dyd, dw.shape, conv, torch.abs))):
+        err = (got.cpu().double() - want).abs()
+        assert bool((err <= 2.0 ** -23 * mag).all()), float((err / mag).max())
 
 
 # filter gradients of small layers, most of which the fp32 GEMM takes: (n, h, w, c, k, r, s, conv)

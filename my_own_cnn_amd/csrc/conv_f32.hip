@@ -35,6 +35,7 @@
 #include "qconv_device.h"
 
 #include <algorithm>
+#include <numeric>
 
 namespace miq {
 namespace {
@@ -1503,6 +1504,14 @@ bool launch_bprop_tile(const Geom& g, const BlockGeom& bg, const float* dy, cons
   const int qb = q % 8 == 0 ? 8 : (q % 4 == 0 ? 4 : (q % 2 == 0 ? 2 : 1));
   const long long z = g.C / (4 * qb);
   if (a.groups >= (1LL << 31) - kDirectThreads || z > 65535) return false;
+  // Where stride and dilation share a factor, one phase in several has all the taps: a fraction of the
+  // workgroups do the work, and with few channels each tap's filter copy and barriers are most of it
+  // (3x3, stride and dilation 2, one-pixel kernel against this: 4 x 28 x 28, 64 -> 64 in 16 groups 8.1 /
+  // 14.2 us, 2 x 112 x 112, 20 -> 36 38 / 50; 32 -> 32 90 / 34).  So it is for one tap on 4 channels of
+  // dx (2 x 112 x 112, 4 -> 64 stride 2 8.6 / 10.2).
+  const bool one_phase = (g.R > 1 && std::gcd(g.dh, g.sh) > 1) || (g.S > 1 && std::gcd(g.dw, g.sw) > 1);
+  if (one_phase && (qb < 8 || g.Kg < 8)) return false;
+  if (g.R * g.S == 1 && qb == 1 && g.Kg >= 64) return false;
   a.fd_rows = fastdiv_m(a.rows);
   a.fd_cgs = fastdiv_m(a.cgs);
   a.fd_sw = fastdiv_m(g.sw);

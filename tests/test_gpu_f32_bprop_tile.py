@@ -20,6 +20,14 @@ CASES = [
     (1, 8, 8, 64, 264, 3, 3, (1, 1, 1, 1, 1, 1, 1)),
     (1, 6, 9, 32, 8, 3, 3, (1, 1, 4, 4, 2, 2, 1)),
     (3, 5, 3, 12, 16, 2, 2, (4, 3, 2, 1, 3, 1, 1)),
+    # on both sides of the rule for strides and dilations with a common factor (the one-pixel kernel
+    # below 8 quads a block or 8 output channels), and for one tap on 4 channels
+    (2, 12, 14, 16, 132, 3, 5, (2, 0, 3, 3, 1, 2, 1)),
+    (2, 11, 13, 16, 16, 3, 3, (2, 2, 2, 2, 2, 2, 1)),
+    (2, 11, 13, 64, 4, 3, 3, (2, 2, 2, 2, 2, 2, 1)),
+    (1, 14, 9, 32, 12, 3, 1, (2, 0, 4, 1, 2, 1, 1)),
+    (1, 14, 9, 20, 64, 1, 1, (0, 0, 2, 2, 1, 1, 1)),
+    (1, 14, 9, 20, 60, 1, 1, (0, 0, 2, 2, 1, 1, 1)),
 ]
 
 

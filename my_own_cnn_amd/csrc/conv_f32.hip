@@ -1370,8 +1370,6 @@ void launch_sum_parts(const float* part, float* dw, long long count, long long n
 
 namespace {
 
-constexpr int kGradFewTaps = 9;  // taps of one workgroup of the split-bf16 dw
-
 // Partial tiles the workspace holds: the implicit GEMM's splits, or, where those are more than half
 // the CUs, up to one per CU for the split-bf16 kernel while 32 MiB hold them (the caller's scratch
 // array of miq_grad_nhwc_f32_noalloc).
@@ -1381,23 +1379,11 @@ long long grad_max_splits(const Geom& g, const BlockGeom& bg) {
   return splits > 128 ? std::max(splits, std::min(256LL, (32LL << 20) / std::max(slice, 1LL))) : splits;
 }
 
-// Whether the split-bf16 dw is the faster one.  With at most one workgroup per CU the fp32 GEMM is
-// bound by the latency of its (at least 8) chunks and takes 21-25 us whatever the layer, or 11 as a
-// single split of at most 64 positions; the split kernel's longer start and tile then lose, by more
-// the more taps and idle columns it computes.  Measured (us, fp32 GEMM against split): 3x3,
-// 8 x 28 x 28, 64 -> 64 25.8 / 28.0 and 128 -> 128 64 / 36; 5x5, 1 x 14 x 14, 64 -> 64 21.6 / 30.6 and
-// 6272 positions 51 / 43; 2x2 29 x 29, 64 -> 64 22.7 / 25.2.  With one tap, or few taps and at most 32
-// output channels (half of the GEMM's tile), the split wins there too: 1x1 21.2 / 12.3 (128 -> 128),
-// 3x3 21.7 / 15.9 (16 -> 16).  Over 628 small layers and blocked layers and 200 drawn ones every call is
-// within 12% of the faster kernel, where the split alone was up to 1.75 times slower.
-bool grad_split_pays(const Geom& g, const BlockGeom& bg, const GradSplit& sp) {
-  const int taps = g.R * g.S;
-  if (taps == 1 || (taps <= kGradFewTaps && g.Kg <= 32)) {
-    return static_cast<long long>(g.N) * bg.bho * bg.bwo > 64 || (taps == 1 && g.Cg > 64);
-  }
-  const long long tiles = ((static_cast<long long>(taps) * g.Cg + kF32BM - 1) / kF32BM) *
+// Workgroups of the ordered fp32 GEMM.
+long long grad_workgroups(const Geom& g, const BlockGeom& bg, const GradSplit& sp) {
+  const long long tiles = ((static_cast<long long>(g.R) * g.S * g.Cg + kF32BM - 1) / kF32BM) *
                           ((g.Kg + kF32BN - 1) / kF32BN) * g.G * static_cast<long long>(bg.By) * bg.Bx;
-  return tiles * sp.splits > 256;
+  return tiles * sp.splits;
 }
 
 }  // namespace
@@ -1409,7 +1395,7 @@ size_t f32_grad_igemm_workspace(const Geom& g, const BlockGeom& bg) {
 }
 
 bool plan_f32_split_grad_igemm(const Geom& g, const BlockGeom& bg, int32_t* tile) {
-  return grad_split_pays(g, bg, grad_split(g, bg, true)) && plan_f32_split_grad(g, bg, grad_max_splits(g, bg), tile);
+  return plan_f32_split_grad(g, bg, grad_max_splits(g, bg), grad_workgroups(g, bg, grad_split(g, bg, true)), tile);
 }
 
 hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw,
@@ -1423,10 +1409,10 @@ hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float
   a.tiles = ((a.kdim + kF32BM - 1) / kF32BM) * a.tn;
   a.gt = a.tiles * g.G * bg.By * bg.Bx;
   const GradSplit sp = grad_split(g, bg, ordered);
-  if (ordered && grad_split_pays(g, bg, sp)) {
+  if (ordered) {
     long long splits = 0;
     hipError_t e;
-    if (launch_f32_split_grad(g, bg, x, dy, dw, ws, grad_max_splits(g, bg), stream, &splits, &e)) {
+    if (launch_f32_split_grad(g, bg, x, dy, dw, ws, grad_max_splits(g, bg), grad_workgroups(g, bg, sp), stream, &splits, &e)) {
       if (e == hipSuccess && splits > 1)
         launch_sum_parts(ws, dw, static_cast<long long>(g.K) * bg.By * bg.Bx * a.kdim, splits, stream);
       return e != hipSuccess ? e : hipGetLastError();

@@ -12,8 +12,10 @@
 // v_mfma_f32_16x16x32_bf16 issue in 0.38 of the time of the eight v_mfma_f32_16x16x4f32 they
 // replace; a loop of them alone sustains 1680 TFLOP/s on this card, 280 of them the convolution's.
 // The matrix core's sums lean towards minus infinity by a part of their last bit (a mean error of 0.3
-// of its rms at K = 576): half of the stages compute on negated filter values, and the running sums
-// change sign with them (a mean of at most 0.04).
+// of its rms at K = 576), so half of the K-blocks compute on negated operands and are subtracted:
+// the second of a stage (stages of 8 octets), every second chunk (of 4: the running sums change sign
+// with it) or stage (blocked dx).  A layer of one chunk keeps its lean in the 4-wave tiles: a sign that
+// turns every few stages cost those 4-7%.
 // What the split does not carry is found at the end of a tile, as a result that is infinite or NaN,
 // and the whole tile is computed again with v_mfma_f32_16x16x4f32: an infinite or NaN input, an
 // input of about 2^105 or more, a scaled sum past the fp32 range (a result of 2^82 or more).
@@ -76,7 +78,6 @@ struct SplitArgs {
   int nchunk;
   int noct;        // R * S * co
   int nst;         // stages per chunk
-  int flip;        // stages between changes of sign
   int ow_taps, ow_cg;  // transposed filter: R * S and channels per group of the original
   int rx, nreg, rh, rw;  // output regions of rh x rw positions, rx per row (forward: the filter blocks)
   int By, Bx, bias_mode;
@@ -112,7 +113,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   constexpr int BU = SO * BN / NT;             // filter (channel, octet) pairs per thread
   constexpr int BSH = 16 / SO;                 // extra slots before every second filter octet
   constexpr int BSZ = 3 * (SO * BN + BSH * SO / 2);  // 16-byte slots of a filter buffer
-  static_assert(BU >= 1 && BU * NT == SO * BN && (SO == 4 || SO == 8), "whole filter stages");
+  static_assert(BU == 1 && NT == SO * BN && (SO == 4 || SO == 8), "whole filter stages, one pair per thread");
   extern __shared__ v4u lds[];
   const Geom& g = a.g;
   const int t = threadIdx.x;
@@ -255,11 +256,12 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       va[j][1] = buffer_load16(rx, left >= 8 ? aoff[j] + 16u : kNone, 4 * c0);
     }
   };
+  float ascale = kSplitScale;  // SO 4: every second chunk's halo is negated
   auto store_a = [&]() {
 #pragma unroll
     for (int j = 0; j < kSplitUnits; ++j) {
       if (aput[j] != ~0u) {
-        const Split8 s = split8(va[j][0], va[j][1], kSplitScale);
+        const Split8 s = split8(va[j][0], va[j][1], ascale);
         v4u* const d = sA + (aput[j] & 0xfffffu);
 #pragma unroll
         for (int p = 0; p < 3; ++p) d[p] = s.p[p];
@@ -362,7 +364,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   };
-  auto store_b = [&](auto set, int buf, float scale) {  // the values of the set's last load_b
+  // the values of the set's last load_b
+  const float bscale = !MULTI && SO == 8 && (boct[0] & 4) ? -kSplitScale : kSplitScale;
+  auto store_b = [&](auto set, int buf, float scale) {
     constexpr int V = MULTI ? decltype(set)::value : 0;
 #pragma unroll
     for (int j = 0; j < BU; ++j) {
@@ -385,8 +389,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
   // steps of up to two segments; a step's fragments are read while the step before it computes.
   // The six products of a step sum from zero, smallest first, and are added to the accumulators.
   int lc = 0, ls = 0;  // stage of the next load_b
-  float scale = kSplitScale;  // of the filter values stored last
-  int left = a.flip;          // stages until the sign turns
   Reach lb;
   set_reach(lb, 0);
   const int first_reach = lb.idx;
@@ -415,11 +417,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     for (int c = 0; c < a.nchunk; ++c) {
       const bool more = c + 1 < a.nchunk;
       for (int s = 0; s < a.nst; ++s) {
-        const bool turn = --left == 0;
-        if (turn) {
-          scale = -scale;
-          left = a.flip;
-        }
         int ao[SO / 4];
 #pragma unroll
         for (int kb = 0; kb < SO / 4; ++kb) ao[kb] = tab[SO * s + 4 * kb + q];
@@ -461,7 +458,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
               }
           }
           if constexpr (st == 0) {
-            store_b(even, buf ^ 1, scale);
+            store_b(even, buf ^ 1, bscale);
             fetch(even);
             if (s == 0) load_a(more ? c + 1 : c);
           }
@@ -469,7 +466,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
           for (int i = 0; i < 2; ++i)
             if (i0 + i < NS) {
 #pragma unroll
-              for (int j = 0; j < 2; ++j) acc[j][i0 + i] += z[j][i];
+              for (int j = 0; j < 2; ++j) acc[j][i0 + i] = kb == 0 ? acc[j][i0 + i] + z[j][i] : acc[j][i0 + i] - z[j][i];
             }
         };
         read(0);
@@ -481,16 +478,17 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
             if constexpr (HALVES > 1) step(std::integral_constant<int, HALVES + 1>{});
           }
         }
-        if (turn) {
+        __syncthreads();
+        buf ^= 1;
+      }
+      if (more) {
+        if constexpr (SO == 4) {
+          ascale = -ascale;
 #pragma unroll
           for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int i = 0; i < NS; ++i) acc[j][i] = -acc[j][i];
         }
-        __syncthreads();
-        buf ^= 1;
-      }
-      if (more) {
         store_a();
         __syncthreads();
       }
@@ -601,7 +599,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
     fetch(even);
     load_a(0);
     if constexpr (MULTI) fetch(odd);
-    store_b(even, 0, scale);
+    store_b(even, 0, MULTI ? kSplitScale : bscale);
     fetch(even);
     store_a();
     __syncthreads();
@@ -695,7 +693,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) f32_split_kernel(SplitArgs a)
       }
     }
   } else {
-    const float unscale = scale < 0.0f ? -kSplitUnscale : kSplitUnscale;
+    const float unscale = ascale < 0.0f ? -kSplitUnscale : kSplitUnscale;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -961,8 +959,8 @@ double igemm_blocked_us(const Geom& g, const BlockGeom& bg, int rh, int rw) {
 // Blocked dx: 16 images (or all of fewer) x a few positions per tile, tiles inside regions of
 // ceil(Ho / By) x ceil(Wo / Bx), so that most reach one filter block.  Variant -1 where the fp32
 // implicit GEMM is the faster kernel: by the two estimates (32 x 14 x 14, 128 -> 64 5x5 in 2 x 2
-// blocks 156 us against 215; over 499 layers no call more than 1.11 times the faster kernel's time
-// but one, where the split alone was up to 1.42), and with one tap unless a filter block serves at
+// blocks 156 us against 215; over 499 layers no call more than 1.11 times the faster kernel's time,
+// where the split alone was up to 1.42), and with one tap unless a filter block serves at
 // most 32 positions: few stages, all latency (16 x 16 x 16, 128 -> 256 in 4 x 4 blocks 20 against 43 us;
 // 512 -> 512 mostly slower, 35 against 48, at best 106 against 90; 16 positions a block 19 against 17).
 SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) {
@@ -994,7 +992,7 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
     }
   }
   // more than 9 taps on full tiles of 16 images take up to 1.7 times their estimate
-  const double margin = g.R * g.S <= 9 ? 1.0 : 0.75;
+  const double margin = g.R * g.S <= 9 ? 1.05 : 0.75;
   if (best.variant >= 0 && !one_tap &&
       split_blocked_us(g, bg, rh, rw, best) > margin * igemm_blocked_us(g, bg, rh, rw)) best.variant = -1;
   return best;
@@ -1044,7 +1042,6 @@ bool launch_f32_split(const Geom& g, const BlockGeom& bg, const float* x, const 
   a.ti = p.ti; a.th = p.th; a.tw = p.tw; a.hh = p.hh; a.hw = p.hw; a.hp = p.hp; a.hps = p.hps;
   a.twp = p.twp; a.ash = p.ash; a.lgh = p.co == 2 ? 0 : (p.co == 4 ? 1 : (p.co == 8 ? 2 : -1));
   a.co = p.co; a.nchunk = p.nchunk; a.noct = p.noct; a.nst = p.nst;
-  a.flip = split_flip(static_cast<long long>(p.nchunk) * p.nst);
   a.ow_taps = g.R * g.S;
   a.ow_cg = g.Kg;
   a.rx = bg.Bx; a.nreg = nreg; a.rh = rh; a.rw = rw;

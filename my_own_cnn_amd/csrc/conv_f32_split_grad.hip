@@ -19,10 +19,10 @@
 // The matrix core's sums lean towards minus infinity by a part of their last bit, which over the
 // K-blocks of a range adds up where rounding errors cancel: every second K-block computes on negated
 // dy and is subtracted.  Relative error of 32 x 56 x 56, 64 -> 64: 4.0e-7 -> 1.3e-7, its mean 0.94 ->
-// 0.00 of its rms; of 32 x 112 x 112 7.4e-7 -> 1.7e-7.  The sign costs a register and a multiply-add in
-// the add's place: 58.4 -> 59.4 us and, 32 x 112 x 112 stride 2, 43.7 -> 44.5; a negation of the sums
-// every few tiles instead took the second to 48, two copies of the tile loop a 2x2 filter from 48 to
-// 283 (spills).
+// 0.00 of its rms; of 32 x 112 x 112 7.4e-7 -> 1.7e-7.  The sign costs nothing measurable (60.7 -> 59 us;
+// 32 x 112 x 112 stride 2, 32 -> 32 43.9 -> 41): it is a wave's in a tile, so staging multiplies by another
+// scalar, and with several wave groups it stays out of the loop.  A negation of the sums every few
+// tiles instead took the second to 48, a tile loop for each sign a 2x2 filter from 48 to 283 (spills).
 //
 // The next tile's values are in flight in registers while a tile computes, and with two LDS buffers
 // (where they fit) they are split and stored under its MFMAs.
@@ -76,6 +76,9 @@ __device__ __forceinline__ v8b join(const v4s& a, const v4s& b) {
 
 // staged dy pairs per thread: 128 positions where wave groups share a tile, else 64
 constexpr int grad_uy(int wk, int wp) { return (wp > 1 ? 128 : 64) * 4 * wk / kGradNT < 1 ? 1 : (wp > 1 ? 128 : 64) * 4 * wk / kGradNT; }
+
+// whether a tile's K-blocks go round its wave groups (yodd in the kernel)
+constexpr bool grad_rotates(int wk, int wc, int wp, int ux) { return wp > 1 && !(wk == 2 && wc == 2) && ux == 3; }
 
 // UX: staged x (position, octet) pairs per thread.  FULL: every workgroup has exactly NB column tiles (taps)
 template <int WK, int WC, int WP, int NB, int CT, int UX, bool FULL>
@@ -193,12 +196,15 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
       vy[j][1] = buffer_load16(ry, yleft >= 8 ? off + 16u : kNone, 0);
     }
   };
-  // dy is staged negated in every second K-block of 32 positions, counted through the tiles, and mma
-  // subtracts those K-blocks' sums
-  static_assert(PY % 64 == 0, "one sign per thread and tile");
-  const float ysign = ((t / OY) >> 5) & 1 ? -kSplitScale : kSplitScale;
+  // dy is staged negated in every second K-block of 32 positions.  One wave group: counted through the
+  // tiles, and mma subtracts those K-blocks' sums.  Several: the odd groups compute the negated
+  // K-blocks and reduce() subtracts their sums; a tile's K-blocks go round the groups from another one
+  // each tile (ROTATE), or stay with them (the instances that spill on the difference).
+  constexpr bool ROTATE = grad_rotates(WK, WC, WP, UX);
+  static_assert(PY % 64 == 0 && 64 % OY == 0 && 64 / OY <= 32, "one sign per wave and tile");
+  const int yodd = (wave * (64 / OY)) >> 5;
   auto store = [&](int buf, int ti_) {
-    const float yscale = ti_ & 1 ? -ysign : ysign;
+    const float yscale = (ROTATE || WP == 1 ? yodd ^ ti_ : yodd) & 1 ? -kSplitScale : kSplitScale;
     char* const bx = reinterpret_cast<char*>(lds) + buf * a.bufsz + xput;
     char* const by = reinterpret_cast<char*>(lds) + buf * a.bufsz + xbytes + yput;
 #pragma unroll
@@ -233,8 +239,7 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
   const unsigned xch = base + 32 * CT * wc + 8 * (n16 & 3);
   const unsigned ych = base + xbytes + 64 * wk + 8 * (n16 & 3);
   auto mma = [&](int buf, int ti_) {
-    for (int kb = wp; kb < a.kbs; kb += WP) {
-      const float sign = (kb ^ ti_) & 1 ? -1.0f : 1.0f;
+    for (int kb = ROTATE ? (wp - ti_) & (WP - 1) : wp; kb < a.kbs; kb += WP) {
       const int m = 32 * kb + 4 * q + (n16 >> 2);
       const unsigned x0 = xch + buf * a.bufsz + tab[m], x1 = xch + buf * a.bufsz + tab[m + 16];
       const unsigned y0 = ych + buf * a.bufsz + m * a.recy, y1 = y0 + 16 * a.recy;
@@ -250,9 +255,14 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
           fx[b & 1][p] = join(lds_read_tr(x0 + toff[b] + 2 * CH * p), lds_read_tr(x1 + toff[b] + 2 * CH * p));
       };
       v4f z[2][2];
-      auto add = [&](int b, int i) {  // acc +- z, one rounding
+      auto add = [&](int b, int i) {
+        if constexpr (WP > 1) {
+          acc[b][i] += z[b & 1][i];
+        } else {  // acc +- z, one rounding
+          const float sign = (kb ^ ti_) & 1 ? -1.0f : 1.0f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[b][i][e] = __builtin_fmaf(z[b & 1][i][e], sign, acc[b][i][e]);
+          for (int e = 0; e < 4; ++e) acc[b][i][e] = __builtin_fmaf(z[b & 1][i][e], sign, acc[b][i][e]);
+        }
       };
       read(0);
 #pragma unroll
@@ -276,8 +286,8 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
       }
     }
   };
-  // the WP wave groups' sums, added in group order into group 0's
-  auto reduce = [&]() {
+  // the WP wave groups' sums, added in group order into group 0's (`negated`: the odd ones subtracted)
+  auto reduce = [&](auto negated) {
     if constexpr (WP > 1) {
       v4f* const r = reinterpret_cast<v4f*>(lds);
 #pragma unroll
@@ -292,7 +302,10 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
 #pragma unroll
           for (int o = 1; o < WP; ++o)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) acc[b][i] += r[(2 * (wave + (o - 1) * WK * WC) + i) * 64 + lane];
+            for (int i = 0; i < 2; ++i) {
+              const v4f v = r[(2 * (wave + (o - 1) * WK * WC) + i) * 64 + lane];
+              acc[b][i] = decltype(negated)::value && (o & 1) ? acc[b][i] - v : acc[b][i] + v;
+            }
         }
       }
     }
@@ -318,7 +331,7 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
     }
     __syncthreads();
   }
-  reduce();
+  reduce(std::true_type{});
 
   bool bad = false;
   if (wp == 0) {
@@ -370,7 +383,7 @@ __global__ void __launch_bounds__(kGradNT, 2) f32_split_grad_kernel(SGradArgs a)
       }
     }
     __syncthreads();
-    reduce();
+    reduce(std::false_type{});
   } else {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -416,11 +429,30 @@ int record_bytes(int channels) {  // an odd multiple of 32 bytes
   return (b / 32) % 2 ? b : b + 32;
 }
 
+// Whether the planned split is the faster kernel.  With at most one workgroup per CU (`gemm` of them)
+// the fp32 GEMM is bound by the latency of its (at least 8) chunks and takes 21-25 us whatever the layer,
+// or 11 as a single split of at most 64 positions; the split kernel's longer start and tile then lose,
+// by more the more taps and idle columns it computes.  Measured (us, fp32 GEMM against split): 3x3,
+// 8 x 28 x 28, 64 -> 64 25.8 / 28.0 and 128 -> 128 64 / 36; 5x5, 1 x 14 x 14, 64 -> 64 21.6 / 30.6 and
+// 6272 positions 51 / 43; 2x2 29 x 29, 64 -> 64 22.7 / 25.2.  Where half of the GEMM's tile would be idle the
+// split wins there too: one tap 21.2 / 12.3 (128 -> 128), few taps and at most 32 output channels 21.7 / 15.9
+// (3x3 16 -> 16); and so it does with few taps and at most 128 positions a split, the GEMM's own
+// number (2 x 14 x 14, 64 -> 64 22.5 / 21.1, 16 -> 64 21.6 / 19.5).  Over 628 small layers and blocked layers
+// and 200 drawn ones every call is within 12% of the faster kernel, where the split alone was up to
+// 1.75 times slower.
+bool grad_pays(const Geom& g, const BlockGeom& bg, const SGradPlan& p, long long gemm) {
+  const int taps = g.R * g.S;
+  const long long positions = static_cast<long long>(g.N) * bg.bho * bg.bwo;
+  if (taps == 1) return positions > 64 || g.Cg > 64;
+  if (taps <= kGradTaps && g.Kg <= 32) return positions > 64;
+  return gemm > 256 || (taps <= kGradTaps && positions > 96 && p.tps * p.kbs <= 4);
+}
+
 // The tile of a launch, or variant -1 where the fp32 implicit GEMM is the faster kernel: more taps
 // than a workgroup takes on a fraction of a 16-channel tile (8 x 224 x 224, 4 -> 64, 7x7 stride 2:
 // 372 against 199 us), and few positions at a stride, whose halos hold four values a position
 // (19 x 13 x 13, 256 -> 64: 30 against 25 us; 8 x 56 x 56, 64 -> 128: 37 against 45).
-SGradPlan grad_plan(const Geom& g, const BlockGeom& bg, long long max_splits) {
+SGradPlan grad_plan(const Geom& g, const BlockGeom& bg, long long max_splits, long long gemm) {
   SGradPlan best{};
   best.variant = -1;
   if (g.Cg % 4 || g.Kg % 4 || g.C % 4 || g.K % 4 || g.dh <= 0 || g.dw <= 0) return best;
@@ -431,6 +463,7 @@ SGradPlan grad_plan(const Geom& g, const BlockGeom& bg, long long max_splits) {
   const int v = g.Kg > 32 ? (g.Cg > 32 ? 0 : 1) : (g.Cg > 32 ? 2 : 3);
   const GradVariant& V = kGradVariants[v];
   const int taps = g.R * g.S;
+  const long long positions = static_cast<long long>(g.N) * bg.bho * bg.bwo;
   SGradPlan p{};
   p.variant = v;
   p.ct_tiles = taps == 1 && g.Cg > 16 * V.wc ? 2 : 1;
@@ -458,6 +491,10 @@ SGradPlan grad_plan(const Geom& g, const BlockGeom& bg, long long max_splits) {
       p.px = p.ti * th * tw;
       p.kbs = (p.px + 31) / 32;
       const long long hp = static_cast<long long>(p.ti) * p.hh * p.hw;
+      // without rotation an odd number of K-blocks per tile leans by one of them, which stays below the
+      // fp32 GEMM's error up to about these sizes
+      const int ux = p.ct_tiles == 2 || taps != kGradTaps || hp * 2 * V.wc > 2 * kGradNT ? 3 : 2;
+      if (V.wp > 1 && !grad_rotates(V.wk, V.wc, V.wp, ux) && (p.kbs & 1) && positions > (p.kbs == 1 ? 1 << 12 : 1 << 20)) continue;
       if (p.hh > 4095 || p.hw > 4095 || p.ti > 126 || hp * (ch / 8) > 3 * kGradNT ||
           32LL * p.kbs * (kr / 8) > grad_uy(V.wk, V.wp) * kGradNT) continue;
       if (static_cast<double>(p.ti) * g.H * g.W * g.C * 4 >= 2147483647.0 ||
@@ -488,7 +525,7 @@ SGradPlan grad_plan(const Geom& g, const BlockGeom& bg, long long max_splits) {
   long long splits = std::max(1LL, std::min({256 / std::max(1LL, std::min(units, 256LL)), best.T, max_splits}));
   best.tps = static_cast<int>((best.T + splits - 1) / splits);
   best.splits = (best.T + best.tps - 1) / best.tps;
-  if (best.splits * units > (1LL << 22) || best.T > (1LL << 30)) best.variant = -1;
+  if (best.splits * units > (1LL << 22) || best.T > (1LL << 30) || !grad_pays(g, bg, best, gemm)) best.variant = -1;
   return best;
 }
 
@@ -514,8 +551,8 @@ hipError_t launch_grad_shape(const SGradArgs& a, const SGradPlan& p, int taps, u
 
 }  // namespace
 
-bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, int32_t* tile) {
-  const SGradPlan p = grad_plan(g, bg, max_splits);
+bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, long long gemm, int32_t* tile) {
+  const SGradPlan p = grad_plan(g, bg, max_splits, gemm);
   if (p.variant < 0) return false;
   const GradVariant& v = kGradVariants[p.variant];
   const int32_t out[8] = {v.wk, v.wc, v.wp, p.ti, p.th, p.tw, p.nbuf, static_cast<int32_t>(p.splits)};
@@ -524,9 +561,10 @@ bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_split
 }
 
 bool launch_f32_split_grad(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw, float* ws,
-                           long long max_splits, hipStream_t stream, long long* splits, hipError_t* err) {
+                           long long max_splits, long long gemm, hipStream_t stream, long long* splits,
+                           hipError_t* err) {
   if (((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15u) != 0) return false;
-  const SGradPlan p = grad_plan(g, bg, max_splits);
+  const SGradPlan p = grad_plan(g, bg, max_splits, gemm);
   if (p.variant < 0) return false;
   SGradArgs a;
   a.x = x; a.dy = dy; a.g = g;

@@ -43,12 +43,6 @@ __device__ __forceinline__ Split8 split8(const v4f& lo, const v4f& hi, float sca
   return out;
 }
 
-// Steps between changes of the sums' sign over `n` steps: an even number of runs of at most 8.
-inline int split_flip(long long n) {
-  const long long runs = 2 * ((n + 15) / 16);
-  return n <= 0 ? 1 : static_cast<int>((n + runs - 1) / runs);
-}
-
 // 16 and 4 bytes at byte offset voff + soff of a buffer; zero where voff is past its 2^31 - 1 bytes
 __device__ __forceinline__ v4f buffer_load16(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
   return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));

@@ -233,12 +233,13 @@ hipError_t launch_f32_grad_igemm(const Geom& g, const BlockGeom& bg, const float
                                  float* ws, bool ordered, hipStream_t stream);
 // The same dw on the bf16 matrix cores (each operand split into three bf16 numbers), with at most
 // max_splits partial tiles in `ws`, which the caller sums in order; one split writes dw.  False
-// when the shape does not fit (nothing is launched).
+// when the shape does not fit or the fp32 GEMM in `gemm` workgroups is faster (nothing is launched).
 bool launch_f32_split_grad(const Geom& g, const BlockGeom& bg, const float* x, const float* dy, float* dw, float* ws,
-                           long long max_splits, hipStream_t stream, long long* splits, hipError_t* err);
+                           long long max_splits, long long gemm, hipStream_t stream, long long* splits,
+                           hipError_t* err);
 // The tile that launch_f32_split_grad takes with aligned tensors, as miq_plan_f32_split's
 // tile[1..8]; false where it takes none.
-bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, int32_t* tile);
+bool plan_f32_split_grad(const Geom& g, const BlockGeom& bg, long long max_splits, long long gemm, int32_t* tile);
 // The tiles of the two above as launch_f32_bprop_igemm and the ordered launch_f32_grad_igemm use them.
 bool plan_f32_split_bprop(const Geom& g, const BlockGeom& bg, int32_t* tile);
 bool plan_f32_split_grad_igemm(const Geom& g, const BlockGeom& bg, int32_t* tile);

@@ -19,8 +19,9 @@
 //   - Two chunks are in flight per thread.  Every pass of the loop issues the same loads:
 //     taps outside the image, values past kdim and rows past M or Kg read a valid address
 //     and are zeroed (or never stored), so the compiler's load counters stay exact.
-//   It serves what the split-bf16 kernel (conv_f32_split.hip) leaves to it: one-tap layers of a
-//   short reduction, few output channels at a stride, dilation below 1.
+//   It serves what the split-bf16 kernel (conv_f32_split.hip) leaves to it by the measured rules of
+//   its plans: one-tap layers of a short reduction or on tiles that do not fill the chip, blocked dx
+//   with many taps, few output channels at a stride, dilation below 1, filters past 32-bit offsets.
 //   The sum order differs from the reference's sequential fp32 loop; results agree within
 //   the reference's own check (verify_tensors with abs 1e-4 / rel 1e-3, main.cpp:306-316).
 //
@@ -36,6 +37,7 @@
 
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 
 namespace miq {
 namespace {
@@ -120,7 +122,11 @@ __device__ __forceinline__ int ceil_div(int a, int d) { return -floor_div(-a, d)
 // BN: channels per workgroup, 64 (128 pixels, waves 4 x 2) or 32 for groups of at most 32
 // output channels (256 pixels, waves 8 x 1; each thread stages two pixel rows, and the waves
 // of threads 256.. load filter rows again without staging them).
-template <int MODE, int BN>
+// SHORT: the MFMA sums restart from zero every 32 reduction values and are added up, so that an
+// error grows with kdim / 32 rather than kdim.  Against 64 bits, 1024 -> 256 1x1: 4.0e-7 relative
+// without, 1.3e-7 with (256 -> 64 2.0e-7 and 0.9e-7; the split kernel 1.2e-7 and 0.7e-7), for 2 to 3%
+// of the time, so only where f32_igemm_launch says.
+template <int MODE, int BN, bool SHORT>
 __global__ void __launch_bounds__(64 * kF32Waves, 1) f32_igemm_kernel(F32Args a) {
   constexpr bool TRANSPOSED = MODE != kFwd;
   constexpr bool MULTI = MODE == kTransBlocked;  // several filter blocks per tile
@@ -401,6 +407,7 @@ __global__ void __launch_bounds__(64 * kF32Waves, 1) f32_igemm_kernel(F32Args a)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // whole groups of P chunks; chunks past the last load the last one again and stage zeros
     for (int c0 = 0; c0 < nch; c0 += P) {
+      v4f z[2][2];  // SHORT: the group's sums
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         const int c = c0 + j;
@@ -413,11 +420,20 @@ __global__ void __launch_bounds__(64 * kF32Waves, 1) f32_igemm_kernel(F32Args a)
 #pragma unroll
           for (int jn = 0; jn < 2; ++jn)
 #pragma unroll
-            for (int im = 0; im < 2; ++im)
-              acc[jn][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(Bf[jn][kk], Af[im][kk], acc[jn][im], 0, 0, 0);
+            for (int im = 0; im < 2; ++im) {
+              v4f& sum = SHORT ? z[jn][im] : acc[jn][im];
+              const v4f from = SHORT && j == 0 && kk == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : sum;
+              sum = __builtin_amdgcn_mfma_f32_16x16x4f32(Bf[jn][kk], Af[im][kk], from, 0, 0, 0);
+            }
         const int jn1 = (j + 1) % P;
         const bool live = c + 1 <= last;
         stage(buf ^ 1, va[jn1], vb[jn1], live ? oka[jn1] : 0u, live && okb[jn1]);
+        if (SHORT && j == P - 1) {
+#pragma unroll
+          for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+            for (int im = 0; im < 2; ++im) acc[jn][im] += z[jn][im];
+        }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       }
     }
@@ -997,8 +1013,8 @@ __global__ void __launch_bounds__(kDirectThreads) f32_grad_direct_kernel(const f
 }
 
 // dw on the fp32 matrix cores, for what the split-bf16 kernel (conv_f32_split_grad.hip) leaves to
-// it (channel counts that are not multiples of 4, unaligned tensors, the float-atomic form, a few
-// shapes it is slower on): dw[g Kg + k][j] = sum over pixels p of dy[p][g Kg + k] * col[p][j],
+// it (channel counts that are not multiples of 4, unaligned tensors, the float-atomic form,
+// small layers that it is slower on): dw[g Kg + k][j] = sum over pixels p of dy[p][g Kg + k] * col[p][j],
 // j = (r, s, ci) the filter column, col the implicit im2col of x.  A workgroup of 8 waves
 // computes 128 columns x 64 channels over its share of the pixels (chunks of 16), with the
 // fprop kernel's staging, fragment layout and pipeline; the pixel range is split over
@@ -1166,7 +1182,11 @@ __global__ void __launch_bounds__(64 * kF32Waves, 1) f32_grad_igemm_kernel(GradA
   for (int j = 0; j < P2; ++j) load(min(j, last), va[j], vb[j], oka[j], okb[j]);
   stage(0, 0, va[0], vb[0], oka[0], true);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // the sums restart every P2 chunks and are added up: the error grows with pixels / 32, not pixels
+  // (8 x 56 x 56, 1024 -> 256 1x1: 3.6e-7 relative without, 1.6e-7 with; 1 x 8 x 8 3x3 0.99e-7 and
+  // 0.75e-7), for 0.4% of the time over 24 layers, at most 1.3%
   for (int c0 = 0; c0 < nch; c0 += P2) {
+    v4f z[2][2];
 #pragma unroll
     for (int j = 0; j < P2; ++j) {
       const int c = c0 + j;
@@ -1180,9 +1200,16 @@ __global__ void __launch_bounds__(64 * kF32Waves, 1) f32_grad_igemm_kernel(GradA
         for (int jn = 0; jn < 2; ++jn)
 #pragma unroll
           for (int im = 0; im < 2; ++im)
-            acc[jn][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(Bf[jn][kk], Af[im][kk], acc[jn][im], 0, 0, 0);
+            z[jn][im] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                Bf[jn][kk], Af[im][kk], j == 0 && kk == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : z[jn][im], 0, 0, 0);
       const int j1 = (j + 1) % P2;
       stage(buf ^ 1, min(c + 1, last), va[j1], vb[j1], oka[j1], c + 1 <= last);
+      if (j == P2 - 1) {
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+          for (int im = 0; im < 2; ++im) acc[jn][im] += z[jn][im];
+      }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
   }
@@ -1624,17 +1651,21 @@ hipError_t f32_igemm_launch(const Geom& g, const BlockGeom& bg, const Regions& r
   a.fd_rx = fastdiv_m(rg.rx);
   const unsigned blocks = static_cast<unsigned>(a.tiles) * static_cast<unsigned>(g.G) *
                           static_cast<unsigned>(rg.ry * rg.rx);
-  const dim3 grid(blocks), block(64 * kF32Waves);
-  if (transposed && a.By * a.Bx > 1) {
-    if (narrow) hipLaunchKernelGGL((f32_igemm_kernel<kTransBlocked, 32>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((f32_igemm_kernel<kTransBlocked, 64>), grid, block, 0, stream, a);
-  } else if (transposed) {
-    if (narrow) hipLaunchKernelGGL((f32_igemm_kernel<kTrans, 32>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((f32_igemm_kernel<kTrans, 64>), grid, block, 0, stream, a);
-  } else {
-    if (narrow) hipLaunchKernelGGL((f32_igemm_kernel<kFwd, 32>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((f32_igemm_kernel<kFwd, 64>), grid, block, 0, stream, a);
-  }
+  // Layers that the split-bf16 kernel holds but is the slower one for: short sums keep their error
+  // near that kernel's.  The bounds are those of its plans (conv_f32_split.hip).
+  const bool blocked_dx = transposed && bg.By * bg.Bx > 1;
+  const bool short_sums = g.R * g.S == 1 ? g.Cg >= (transposed ? 128 : 256) : blocked_dx;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kF32Waves), 0, stream, a);
+  };
+  auto launch_mode = [&](auto mode) {
+    constexpr int kMode = decltype(mode)::value;
+    if (narrow) launch(short_sums ? f32_igemm_kernel<kMode, 32, true> : f32_igemm_kernel<kMode, 32, false>);
+    else launch(short_sums ? f32_igemm_kernel<kMode, 64, true> : f32_igemm_kernel<kMode, 64, false>);
+  };
+  if (blocked_dx) launch_mode(std::integral_constant<int, kTransBlocked>{});
+  else if (transposed) launch_mode(std::integral_constant<int, kTrans>{});
+  else launch_mode(std::integral_constant<int, kFwd>{});
   return hipGetLastError();
 }
 }  // namespace

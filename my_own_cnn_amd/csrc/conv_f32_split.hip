@@ -821,18 +821,22 @@ void consider(const Geom& g, int rh, int rw, long long nreg, int v, int ti, int 
   }
 }
 
-// One tap: whether the split is the faster kernel in the chosen tile (us, fp32 GEMM against split).
-// Each stage is as long as the latency of its filter values, so it has to hold 8 octets: tiles of 4
-// waves hold 4 a stage (1x1 32 x 14 x 14, 256 -> 64 15.8 / 17.0, until 512 channels: 8 x 14 x 14,
-// 128 -> 512 dx 30.2 / 27.1), and 256 positions leave room for fewer than 8 octets of halo (112 x 112,
-// 256 -> 16 17.8 / 22.4; dx over more than 256 workgroups 33.0 / 29.1).  A last round of few workgroups
-// is a whole one (8 x 72 x 72, 96 -> 128 dx in 352: 25.3 / 28.0).  Of 803 layers no call is more than 1.12
-// times the faster kernel's time, where the split alone was up to 1.27 (blocked forward, 256 -> 32).
+// One tap: whether the split is the faster kernel in the chosen tile (us, fp32 GEMM against split; the
+// GEMM is taken where it gains more than the 2 to 4% that its short sums cost).  Each stage is as long
+// as the latency of its filter values, so it has to hold 8 octets or the reduction 256 channels: tiles
+// of 4 waves hold 4 a stage (dx 8 x 56 x 56, 64 -> 128 11.3 / 12.0; 8 x 28 x 28, 256 -> 256 18.0 /
+// 16.5), and 256 positions leave room for fewer than 8 octets of halo (112 x 112, 256 -> 16 17.8 /
+// 22.4), which pays while its second round is not full (32 x 56 x 56 2 x 2 blocks, 512 -> 32 54.9 /
+// 49.0).  A last round of few workgroups is a whole one (dx 8 x 72 x 72, 96 -> 128 in 352: 25.3 / 28.0;
+// 96 -> 256 42.1 / 40.2).
 bool one_tap_pays(const Geom& g, const SplitPlan& p, bool transposed) {
   const SplitVariant& v = kVariants[p.variant];
-  if (v.wm < 4) return g.Cg >= 512;
-  if (v.wn == 1) return p.nchunk * p.nst <= (g.Cg + 63) / 64 || (transposed && p.blocks > 256);
-  return v.nseg == 1 || p.blocks <= 256 || 256.0 * ((p.blocks + 255) / 256) <= 1.35 * static_cast<double>(p.blocks);
+  if (v.wn == 1) {
+    return p.nchunk * p.nst <= (g.Cg + 63) / 64 || (p.blocks > 256 && (transposed || p.blocks <= 512));
+  }
+  if (g.Cg >= 256 || v.nseg == 1) return true;
+  return v.wm == 4 &&
+         (p.blocks <= 256 || 256.0 * ((p.blocks + 255) / 256) <= 1.35 * static_cast<double>(p.blocks));
 }
 
 // The tile of a launch, or variant -1 where the fp32 implicit GEMM is the faster kernel (measured
@@ -932,7 +936,7 @@ Reach1 worst_reach(int in, int nreg, int rlen, int step, int len, int blk, int R
 // Estimated microseconds of the blocked dx: both kernels wait for their worst tile, whose pieces
 // (stages of the split kernel, 16-channel chunks of the fp32 GEMM) pass one after the other.  Fitted to
 // 422 layers of 1 x 2 to 4 x 4 blocks, 1 to 32 images, 3x3 and 5x5 taps: the GEMM within 4% on
-// average, the split within 11%.
+// average (its short sums 3% on top), the split within 11%.
 double split_blocked_us(const Geom& g, const BlockGeom& bg, int rh, int rw, const SplitPlan& p) {
   const Reach1 a = worst_reach(g.H, bg.By, rh, p.th, p.th, bg.bho, g.R, g.dh, g.ph);
   const Reach1 b = worst_reach(g.W, bg.Bx, rw, p.tw, p.tw, bg.bwo, g.S, g.dw, g.pw);
@@ -953,23 +957,32 @@ double igemm_blocked_us(const Geom& g, const BlockGeom& bg, int rh, int rw) {
                           : worst_reach(g.W, bg.Bx, rw, rw, rw, bg.bwo, g.S, g.dw, g.pw);
   const double chunks = static_cast<double>(a.taps) * b.taps * g.Cg / 16;
   const double tiles = std::ceil(static_cast<double>(g.N) * rh * rw / bm) * bg.By * bg.Bx * ((g.Kg + bn - 1) / bn) * g.G;
-  return 12.1 + 0.832 * chunks * std::max(1.0, tiles / 256);
+  return 12.1 + 0.857 * chunks * std::max(1.0, tiles / 256);
+}
+
+// Blocked dx with one tap: whether the split is the faster kernel in the chosen tile (us, fp32 GEMM
+// against split).  Few stages, all latency: small tiles, or tiles of 256 positions of few images that
+// fill a round (two of a longer reduction) where the GEMM's tiles take twice as many.
+// 32 x 8 x 8, 256 -> 256 in 4 x 4 blocks 20.4 / 18.0; 8 x 28 x 28, 512 -> 256 in 2 x 2 33.4 / 29.6;
+// 8 x 56 x 56, 256 -> 256 59.2 / 56.5, 512 -> 256 99 / 109; 32 x 16 x 16, 512 -> 256 in tiles of 16
+// images 33.5 / 45.0; 1 x 28 x 28, 256 -> 256 20.1 / 25.2.
+bool one_tap_blocked_pays(const Geom& g, const BlockGeom& bg, const SplitPlan& p) {
+  if (static_cast<long long>(g.N) * bg.bho * bg.bwo <= 32 || (p.th * p.tw <= 4 && p.ti <= 8)) return true;
+  return p.variant == 0 && p.ti <= 4 && p.blocks >= 192 && p.blocks <= (g.Cg >= 256 ? 512 : 256);
 }
 
 // Blocked dx: 16 images (or all of fewer) x a few positions per tile, tiles inside regions of
 // ceil(Ho / By) x ceil(Wo / Bx), so that most reach one filter block.  Variant -1 where the fp32
 // implicit GEMM is the faster kernel: by the two estimates (32 x 14 x 14, 128 -> 64 5x5 in 2 x 2
 // blocks 156 us against 215; over 499 layers no call more than 1.11 times the faster kernel's time,
-// where the split alone was up to 1.42), and with one tap unless a filter block serves at
-// most 32 positions: few stages, all latency (16 x 16 x 16, 128 -> 256 in 4 x 4 blocks 20 against 43 us;
-// 512 -> 512 mostly slower, 35 against 48, at best 106 against 90; 16 positions a block 19 against 17).
+// where the split alone was up to 1.42), and with one tap by one_tap_blocked_pays.
 SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) {
   SplitPlan best{};
   best.variant = -1;
   const long long nreg = static_cast<long long>(bg.By) * bg.Bx;
   if (!plain_extents(g) || g.dh <= 0 || g.dw <= 0 || g.R > 16 || g.S > 16) return best;
   const bool one_tap = g.R * g.S == 1;
-  if (one_tap && (g.Cg < 128 || static_cast<long long>(g.N) * bg.bho * bg.bwo > 32)) return best;
+  if (one_tap && g.Cg < 128) return best;
   if (static_cast<double>(g.Kg) * nreg * g.R * g.S * g.Cg * 4 >= 2147483647.0) return best;
   for (int v = 0; v < static_cast<int>(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
     if ((kVariants[v].wn == 1) != (g.Kg <= 32) || kVariants[v].nseg == 1) continue;
@@ -993,8 +1006,9 @@ SplitPlan make_blocked_plan(const Geom& g, const BlockGeom& bg, int rh, int rw) 
   }
   // more than 9 taps on full tiles of 16 images take up to 1.7 times their estimate
   const double margin = g.R * g.S <= 9 ? 1.05 : 0.75;
-  if (best.variant >= 0 && !one_tap &&
-      split_blocked_us(g, bg, rh, rw, best) > margin * igemm_blocked_us(g, bg, rh, rw)) best.variant = -1;
+  if (best.variant >= 0 &&
+      !(one_tap ? one_tap_blocked_pays(g, bg, best)
+                : split_blocked_us(g, bg, rh, rw, best) <= margin * igemm_blocked_us(g, bg, rh, rw))) best.variant = -1;
   return best;
 }
 

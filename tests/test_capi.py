@@ -422,14 +422,20 @@ def test_plan_f32_split_names_the_tile_of_the_split_kernels():
 # (op, (n, h, w, c, r, s, k), blocks, whether the pass computes on split operands)
 SPLIT_ROUTES = [
     ("fprop", (1, 56, 56, 256, 1, 1, 64), 1, True),
-    ("fprop", (32, 14, 14, 256, 1, 1, 64), 1, False),   # 4 waves a tile, 4 octets a stage
+    ("fprop", (32, 14, 14, 256, 1, 1, 64), 1, True),    # 4 waves a tile, but 256 channels
+    ("bprop", (8, 56, 56, 64, 1, 1, 128), 1, False),    # 4 waves a tile, 4 octets a stage
     ("fprop", (1, 112, 112, 256, 1, 1, 16), 1, False),  # 256 positions, fewer than 8 octets of halo
     ("fprop", (8, 16, 16, 256, 1, 1, 32), 2, False),
     ("fprop", (32, 56, 56, 256, 1, 1, 128), 1, True),
-    ("bprop", (8, 14, 14, 128, 1, 1, 512), 1, True),    # 4 waves, but 512 channels
+    ("fprop", (32, 56, 56, 512, 1, 1, 32), 2, True),    # the same, a second round in part
+    ("fprop", (32, 72, 72, 256, 1, 1, 32), 1, False),   # three rounds
+    ("bprop", (8, 14, 14, 128, 1, 1, 512), 1, True),
     ("bprop", (8, 72, 72, 96, 1, 1, 128), 1, False),    # a round and a third
     ("bprop", (16, 16, 16, 128, 1, 1, 256), 4, False),  # blocked, one tap
     ("bprop", (1, 16, 16, 128, 1, 1, 256), 4, True),    # 16 positions a block
+    ("bprop", (32, 8, 8, 256, 1, 1, 256), 4, True),     # tiles of 4 positions of 8 images
+    ("bprop", (8, 28, 28, 512, 1, 1, 256), 2, True),    # one full round of few images
+    ("bprop", (32, 16, 16, 512, 1, 1, 256), 2, False),  # 16 images a tile
     ("bprop", (32, 14, 14, 128, 5, 5, 64), 2, False),   # 16 images, 25 taps
     ("bprop", (1, 14, 14, 128, 5, 5, 64), 2, True),
     ("bprop", (32, 56, 56, 64, 3, 3, 64), 4, True),

@@ -238,3 +238,54 @@ def test_fp32_grad_auto_is_deterministic(device, case):
     assert np.abs(want).max() < 2 ** 24
     for kw in ({}, {"workspace": ws}, {"algo": "atomic"}):
         np.testing.assert_array_equal(grad(xi, dyi, **kw).view(np.uint32), want.view(np.uint32), err_msg=f"{name} {kw}")
+
+
+SHORT_SUMS = [
+    # pass, n, h, w, c, k, taps, blocks; reductions that end inside a chunk or between the two of a pair
+    ("fprop", 1, 96, 96, 1028, 16, 1, 1),
+    ("fprop", 1, 96, 96, 1040, 32, 1, 1),
+    ("bprop", 1, 64, 64, 32, 996, 1, 1),
+    ("bprop", 4, 16, 16, 68, 1024, 1, 4),
+    ("bprop", 32, 14, 14, 128, 68, 5, 2),
+    ("grad", 1, 7, 9, 64, 64, 5, 1),
+    ("grad", 2, 16, 12, 64, 64, 3, 2),
+]
+
+
+@pytest.mark.parametrize("case", SHORT_SUMS, ids=str)
+def test_fp32_igemm_sums_restart(device, case):
+    """Reductions of K values on the fp32 MFMA kernel where it stands in for the split-bf16 one: sums of
+    32 values that are then added.  Of independent terms a partial sum of j of K values has j / K of the
+    result's variance, and a rounding's variance is at most a third of 2^-48 of its square.  With a
+    rounding per value, the groups add (1 + 2 + .. + 32) / 32 = 16.5 such thirds and their K / 32 sums
+    K / 64; a single chain has K / 2 instead (measured at K = 1024: 1.3e-7 and 4.0e-7)."""
+    op, n, h, w, c, k, t, b = case
+    rng = np.random.default_rng(41)
+    draw = lambda *size: torch.from_numpy(rng.standard_normal(size).astype(np.float32)).to(device)
+    x, dy = draw(n, h, w, c), draw(n, h, w, k)
+    wt = draw(k, b, b, t, t, c)
+    p = M.BlockConv2DParams(M.Conv2DParams(t // 2, t // 2, 1, 1, 1, 1, 1), b, b)
+    dims = (n, h, w, c, t, t, k)
+    assert M.plan_f32_split(op, *dims, p) is None
+    xp = torch.nn.functional.pad(x.double(), (0, 0, t // 2, t // 2, t // 2, t // 2))
+    want = torch.zeros(dict(fprop=dy, bprop=xp, grad=wt)[op].shape, dtype=torch.float64, device=device)
+    for by in range(b):
+        for bx in range(b):
+            ys, xs = (slice(i * e // b, (i + 1) * e // b) for i, e in ((by, h), (bx, w)))
+            for r in range(t):
+                for s in range(t):
+                    yr, xr = slice(ys.start + r, ys.stop + r), slice(xs.start + s, xs.stop + s)
+                    f, d, i = wt[:, by, bx, r, s].double(), dy[:, ys, xs].double(), xp[:, yr, xr]
+                    if op == "fprop": want[:, ys, xs] += i @ f.T.contiguous()
+                    elif op == "bprop": want[:, yr, xr] += d @ f
+                    else: want[:, by, bx, r, s] += d.reshape(-1, k).T.contiguous() @ i.reshape(-1, c)
+    if op == "fprop": got = torch.empty_like(dy); M.launch_block_fprop_nhwc(x, wt, got, *dims, p, None)
+    elif op == "bprop":
+        got = torch.empty_like(x); M.launch_block_bprop_nhwc(dy, wt, got, *dims, p)
+        want = want[:, t // 2:t // 2 + h, t // 2:t // 2 + w]
+    else: got = torch.empty_like(wt); M.launch_block_grad_nhwc(x, dy, got, *dims, p)
+    torch.cuda.synchronize()
+    terms = dict(fprop=c, bprop=k * t * t, grad=n * h * w // (b * b))[op]
+    bound = 2.0 ** -24 * ((16.5 + terms / 64) / 3) ** 0.5
+    error = float((got.double() - want).norm() / want.norm())
+    assert error <= bound, (error, bound)

@@ -815,7 +815,7 @@ __global__ void __launch_bounds__(kDirectThreads) f32_bprop_direct4_kernel(const
 // run the same taps.  Per tap the workgroup copies the filter slice of its 4 QB channels, kTileKo
 // output channels at a time, to LDS; dy is read as float4s of 4 output channels.  Per 4 output
 // channels a thread issues 8 loads for 128 multiplies and adds; the one-pixel kernel above issues
-// 8 for 32 and is bound by them: 32 x 112 x 112 stride 2, 32 -> 32 281 -> 61 us; 8 x 56 x 56,
+// 8 for 32 and is bound by them: 32 x 112 x 112 stride 2, 32 -> 32 271 -> 64 us; 8 x 56 x 56,
 // 128 -> 128 347 -> 71; 8 x 224 x 224 7x7, 4 -> 64 1417 -> 780.  Bound by the vector ALU now: one
 // multiply and one add per term, not contracted, are 51 us of the first at 2.2 GHz.
 constexpr int kTilePix = 4;

@@ -31,9 +31,9 @@
 // The next stage's filter values and the next chunk's halo are in flight in registers while a
 // stage's MFMAs run.
 //
-// Measured (us; before: the fp32 implicit GEMM of conv_f32.hip): 32 x 56 x 56, 64 -> 64 3x3 54-58
-// (110), its dx 58 (122); 32 x 28 x 28, 128 -> 256 97 (207), dx 97 (226), 2 x 4 filter blocks 93
-// (199); 16 x 64 x 64 dilated 32 (57); four groups of 32 64 (111); one 56 x 56 image 13.1 (30.8).
+// Measured (us, back to back; before: the fp32 implicit GEMM of conv_f32.hip): 32 x 56 x 56, 64 -> 64
+// 3x3 59 (106), its dx 59 (118); 32 x 28 x 28, 128 -> 256 100 (198), dx 95 (218), 2 x 4 filter blocks
+// 102 (199); 16 x 64 x 64 dilated 34 (59); four groups of 32 70 (115); one 56 x 56 image 12.8 (30.8).
 // Few tiles are bound by the stages' latency: 8 waves on 16 positions each (NSEG 1) halve the
 // stages of 4 waves on 32 (one image 15.4 -> 13.1, 4 x 16 x 16, 256 -> 64 42 -> 38).
 // Bound by the matrix instructions and the power they draw: with everything but the MFMAs and
@@ -96,8 +96,8 @@ __device__ __forceinline__ int f32s_slot(int row, int g) { return 4 * row + (g ^
 // segments skipping the taps that none of its lanes uses.  With the image the fastest index of a
 // tile (16 images: a segment is one position) nearly every tap of a segment falls in one block.
 // Measured (us; before: the fp32 implicit GEMM's blocked form): 32 x 28 x 28, 128 -> 256 in 2 x 4
-// blocks 216 (366); 32 x 56 x 56, 64 -> 64 in 2 x 2 119 (123), in 4 x 4 117 (155); one image in
-// 4 x 4 38 (78). The stages of a neighbour's few taps bound it: a stage's filter values cost the
+// blocks 215 (368); 32 x 56 x 56, 64 -> 64 in 2 x 2 125 (127), in 4 x 4 119 (158); one image in
+// 4 x 4 44 (80). The stages of a neighbour's few taps bound it: a stage's filter values cost the
 // same whatever its MFMAs, so fetching them two stages ahead and keeping the reach in LDS (five
 // divisions a block otherwise) took the first from 404 to 226.
 enum SplitMode : int { kSplitFwd = 0, kSplitTrans = 1, kSplitTransBlocked = 2 };

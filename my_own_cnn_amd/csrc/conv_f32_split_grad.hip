@@ -28,12 +28,14 @@
 // (where they fit) they are split and stored under its MFMAs.
 //
 // Measured (us, the split sums' pass apart; before: the fp32 implicit GEMM): 32 x 56 x 56, 64 -> 64
-// 3x3 54 (197); 32 x 28 x 28, 128 -> 256 102 with 2 x 4 blocks (374); 32 x 112 x 112 stride 2,
-// 32 -> 32 40 (123); four groups of 32 63. Error against 64 bits 3.0e-7 -> 0.8e-7 (one 56 x 56
-// layer). Bound by the MFMAs and their fragment reads (48 of the 63 us of an earlier build, 34 at
+// 3x3 51 (197); 32 x 28 x 28, 128 -> 256 98 with 2 x 4 blocks (374); 32 x 112 x 112 stride 2,
+// 32 -> 32 39 (123); four groups of 32 68 with the sums (504). Error against 64 bits 3.0e-7 -> 0.8e-7
+// (one 56 x 56 layer). Bound by the MFMAs and their fragment reads (48 of the 63 us of an earlier build, 34 at
 // the bare rate), the rest is the loads' and the split's issue. Registers decide: 72 accumulators,
 // 48 fragments and 24 to 40 values in flight leave none over, and each pair fewer in flight bought
-// 5-9 us through the spills it saved.
+// 5-9 us through the spills it saved.  What still spills (of 256 registers a wave): with 9 columns and 2
+// pairs of x in flight 1 (2 x 4 x 1), 16 (2 x 2 x 2) and 4 (the other two), with 3 pairs 13, 60, 21 and
+// 23, with a count of taps other than 9 29, 59, 28 and 30; the smaller instances none.
 
 #include "f32_split.h"
 

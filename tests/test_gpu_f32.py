@@ -241,14 +241,18 @@ def test_fp32_grad_auto_is_deterministic(device, case):
 
 
 SHORT_SUMS = [
-    # pass, n, h, w, c, k, taps, blocks; reductions that end inside a chunk or between the two of a pair
-    ("fprop", 1, 96, 96, 1028, 16, 1, 1),
-    ("fprop", 1, 96, 96, 1040, 32, 1, 1),
-    ("bprop", 1, 64, 64, 32, 996, 1, 1),
-    ("bprop", 4, 16, 16, 68, 1024, 1, 4),
-    ("bprop", 32, 14, 14, 128, 68, 5, 2),
-    ("grad", 1, 7, 9, 64, 64, 5, 1),
-    ("grad", 2, 16, 12, 64, 64, 3, 2),
+    # pass, n, h, w, c, k, taps, blocks, dilation; reductions that end inside a chunk or between two chunks of
+    # a pair, on tiles of 32 and 64 channels of each pass (the split kernel takes no dilation of 0)
+    ("fprop", 1, 96, 96, 1028, 16, 1, 1, 1),
+    ("fprop", 1, 96, 96, 1040, 32, 1, 1, 1),
+    ("fprop", 1, 24, 24, 516, 72, 1, 1, 0),
+    ("bprop", 1, 64, 64, 32, 996, 1, 1, 1),
+    ("bprop", 8, 56, 56, 64, 196, 1, 1, 1),
+    ("bprop", 4, 16, 16, 68, 1024, 1, 4, 1),
+    ("bprop", 2, 32, 32, 28, 324, 1, 2, 1),
+    ("bprop", 32, 14, 14, 128, 68, 5, 2, 1),
+    ("grad", 1, 7, 9, 64, 64, 5, 1, 1),
+    ("grad", 2, 16, 12, 64, 64, 3, 2, 1),
 ]
 
 
@@ -259,12 +263,12 @@ def test_fp32_igemm_sums_restart(device, case):
     result's variance, and a rounding's variance is at most a third of 2^-48 of its square.  With a
     rounding per value, the groups add (1 + 2 + .. + 32) / 32 = 16.5 such thirds and their K / 32 sums
     K / 64; a single chain has K / 2 instead (measured at K = 1024: 1.3e-7 and 4.0e-7)."""
-    op, n, h, w, c, k, t, b = case
+    op, n, h, w, c, k, t, b, dil = case
     rng = np.random.default_rng(41)
     draw = lambda *size: torch.from_numpy(rng.standard_normal(size).astype(np.float32)).to(device)
     x, dy = draw(n, h, w, c), draw(n, h, w, k)
     wt = draw(k, b, b, t, t, c)
-    p = M.BlockConv2DParams(M.Conv2DParams(t // 2, t // 2, 1, 1, 1, 1, 1), b, b)
+    p = M.BlockConv2DParams(M.Conv2DParams(t // 2, t // 2, 1, 1, dil, dil, 1), b, b)
     dims = (n, h, w, c, t, t, k)
     assert M.plan_f32_split(op, *dims, p) is None
     xp = torch.nn.functional.pad(x.double(), (0, 0, t // 2, t // 2, t // 2, t // 2))
